@@ -209,6 +209,7 @@ def _hc_inputs(c, seed):
 
 
 def prepare(case, seed):
+    ops.load_extension()              # once per process, as a program does at its start
     if case["op"] == "hc":
         return dict(case, x=_hc_inputs(case, seed))
     if case["op"] == "moe":
