@@ -120,10 +120,10 @@ def _err_flag(device):
     i = device.index if device.index is not None else torch.cuda.current_device()
     f = _err_flags.get(i)
     if f is None:
+        load_extension()  # before the lock: it takes the same one
         with _lock:
             f = _err_flags.get(i)
             if f is None:
-                load_extension()
                 addr = torch.ops.sa_amd.index_error_flag_address(i)
                 f = _err_flags[i] = ctypes.c_int32.from_address(addr)
     return f

@@ -10,6 +10,8 @@
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -460,3 +462,18 @@ def test_supported_head_counts_validate(libs, h):
         assert ws.value >= ws16.value + 2 * a.b * a.m * 16 * 512 * 2
     else:
         assert ws.value == ws16.value
+
+
+def test_first_call_of_a_process_does_not_wait_for_itself():
+    """The deferred index check is the first thing a call does, so in a fresh
+    process its flag lookup is also what loads the extension; the two take the
+    same lock. Without a GPU the lookup then raises; it must not hang."""
+    code = ("import sys; sys.path.insert(0, sys.argv[1]); import torch, submission\n"
+            "try:\n"
+            "    submission._err_flag(torch.device('cuda', 0))\n"
+            "except RuntimeError:\n"
+            "    pass\n"
+            "assert submission._loaded\n")
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       "kernelgen-challenge_amd")
+    subprocess.run([sys.executable, "-c", code, pkg], check=True, timeout=300)
