@@ -348,15 +348,18 @@ struct PlanParams {
   const int32_t* ids;
   int32_t* eoff;      // [E + 1] first sorted position of each expert
   int32_t* sorted;    // [P] pair ids (t * topk + slot) grouped by expert
-  int32_t* tiles;     // [0] = tile count, then int4 (expert, start, rows, 0) per tile
+  int32_t* tiles;     // [0] = tile count, [1] = tiles before the small ones (of all
+                      // with split_small = 0), then int4 (expert, start, rows, 0) per tile
   int64_t P;
   int E, tile_rows;
+  int split_small;    // list the tiles of at most tile_rows / 2 pairs last
 };
 
 struct PlanSmem {
   int cnt[kMaxExperts];
   int off[kMaxExperts + 1];
   int toff[kMaxExperts + 1];
+  int soff[kMaxExperts + 1];
   int cur[kMaxExperts];
 };
 
@@ -365,6 +368,11 @@ __device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
   int* s_cnt = sm.cnt;
   int* s_off = sm.off;
   int* s_toff = sm.toff;
+  int* s_soff = sm.soff;
+  // an expert's last tile goes into the list of small ones
+  auto small_tile = [&](int n) {
+    return p.split_small && n % p.tile_rows > 0 && n % p.tile_rows <= p.tile_rows / 2;
+  };
   int* s_cur = sm.cur;
   const int tid = threadIdx.x;
   for (int e = tid; e < kMaxExperts; e += 1024) {
@@ -375,36 +383,45 @@ __device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
   for (int64_t i = tid; i < p.P; i += 1024) atomicAdd(&s_cnt[p.ids[i]], 1);
   __syncthreads();
   if (tid < 64) {  // exclusive scans of counts and tile counts over <= 256 experts
-    int carry = 0, tcarry = 0;
+    int carry = 0, tcarry = 0, scarry = 0;
     for (int c = 0; c < kMaxExperts / 64; ++c) {
       const int e = 64 * c + tid;
       const int v = e < p.E ? s_cnt[e] : 0;
-      const int tv = (v + p.tile_rows - 1) / p.tile_rows;
-      int incl = v, tincl = tv;
+      const int sv = small_tile(v) ? 1 : 0;
+      const int tv = (v + p.tile_rows - 1) / p.tile_rows - sv;
+      int incl = v, tincl = tv, sincl = sv;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int a = __shfl_up(incl, o);
         const int b = __shfl_up(tincl, o);
+        const int d = __shfl_up(sincl, o);
         if (tid >= o) {
           incl += a;
           tincl += b;
+          sincl += d;
         }
       }
       if (e < p.E) {
         s_off[e] = carry + incl - v;
         s_toff[e] = tcarry + tincl - tv;
+        s_soff[e] = scarry + sincl - sv;
       }
       carry += __shfl(incl, 63);
       tcarry += __shfl(tincl, 63);
+      scarry += __shfl(sincl, 63);
     }
     if (tid == 0) {
       s_off[p.E] = carry;
       s_toff[p.E] = tcarry;
+      s_soff[p.E] = scarry;
     }
   }
   __syncthreads();
   for (int e = tid; e <= p.E; e += 1024) p.eoff[e] = s_off[e];
-  if (tid == 0) p.tiles[0] = s_toff[p.E];
+  if (tid == 0) {
+    p.tiles[0] = s_toff[p.E] + s_soff[p.E];
+    p.tiles[1] = s_toff[p.E];
+  }
   for (int64_t i = tid; i < p.P; i += 1024) {
     const int e = p.ids[i];
     p.sorted[s_off[e] + atomicAdd(&s_cur[e], 1)] = int32_t(i);
@@ -412,7 +429,9 @@ __device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
   for (int e = tid; e < p.E; e += 1024) {
     const int n = s_cnt[e];
     for (int k = 0; k * p.tile_rows < n; ++k) {
-      int32_t* tl = p.tiles + 4 + 4 * (s_toff[e] + k);
+      const bool last = (k + 1) * p.tile_rows >= n;
+      const int at = last && small_tile(n) ? s_toff[p.E] + s_soff[e] : s_toff[e] + k;
+      int32_t* tl = p.tiles + 4 + 4 * at;
       tl[0] = e;
       tl[1] = s_off[e] + k * p.tile_rows;
       tl[2] = min(p.tile_rows, n - k * p.tile_rows);
@@ -480,7 +499,7 @@ struct GemmParams {
   int topk;
   int col_tiles;         // output-column tiles per pair tile
   int ct_per_wg;         // column tiles one work-group runs (fm_stream_kernel)
-  int xcd_grid;          // large/big tiles: the 2 x 4 XCD grid of xcd_item
+  int xcd_grid;          // large tiles: the 2 x 4 XCD grid of xcd_item
   // GEMM 2 with topk <= 2 (fm_stream_kernel): add each pair's bf16 row into
   // the token's output row instead of writing yw (null: write yw)
   __bf16* fsum;
@@ -498,23 +517,18 @@ __device__ __forceinline__ void add_bf16x2(__bf16* out, __bf16 a0, __bf16 a1) {
   asm volatile("global_atomic_pk_add_bf16 %0, %1, off sc1" : : "v"(out), "v"(v) : "memory");
 }
 
-// Work item (pair tile, column tile) of a large or big GEMM work-group.
-// Work-group b runs on XCD b % 8 (dispatch is round-robin over the XCDs, in
-// order of b). Plainly, b -> (b / col_tiles, b % col_tiles): column tile c of
-// every pair tile runs on XCD c % 8, so a weight tile is read into one L2 and
-// shared there by the pair tiles of its expert, while every pair tile's
-// gathered A rows are read into col_tiles L2s. With p.xcd_grid the XCDs form
-// a 2 x 4 grid instead: XCD x takes the column tiles of half x % 2 of every
-// pair tile in its contiguous quarter x / 2 of the tile table, pair tile by
-// pair tile, so a pair tile's A rows go to two L2s, and an expert's pair
-// tiles (adjacent in the table) still share its weight rows in one L2.
-// The host sets xcd_grid when experts average fewer than two pair tiles and
-// the items outnumber the CUs. Measured at K = 2048, N = 1024 (gate-up +
-// down): M = 4096, E = 64, topk = 6 (1.5 pair tiles per expert) 5-10 %
-// faster; M = 512-3072 at E = 64, 1-7 %; but M = 4096, E = 8, topk = 2 (4
-// pair tiles per expert) 20 % slower with one set of routings and level with
-// another, and M = 8192, E = 8 8 % slower. Whole column tiles on each XCD
-// (an 8 x 1 grid) gained 10 % at M = 4096, E = 64 and lost 15 % at E = 8.
+// Work item (pair tile, column tile) of a large GEMM work-group. Work-group b
+// runs on XCD b % 8 (dispatch is round-robin over the XCDs, in order of b).
+// Plainly, b -> (b / col_tiles, b % col_tiles): column tile c of every pair
+// tile runs on XCD c % 8, so a weight tile is read into one L2 and shared
+// there by the pair tiles of its expert, while every pair tile's gathered A
+// rows are read into col_tiles L2s. With p.xcd_grid the XCDs form a 2 x 4 grid
+// instead: XCD x takes the column tiles of half x % 2 of every pair tile in
+// its contiguous quarter x / 2 of the tile table, pair tile by pair tile, so a
+// pair tile's A rows go to two L2s, and an expert's pair tiles (adjacent in
+// the table) still share its weight rows in one L2. The host sets xcd_grid
+// when experts average fewer than two pair tiles and the items outnumber the
+// CUs (1-7 % faster at M = 512-3072, E = 64, topk = 6, K = 2048, N = 1024).
 // False: no item for this work-group.
 constexpr int kXcds = 8;
 constexpr int kXcdColGroups = 2;
@@ -733,185 +747,305 @@ __global__ void __launch_bounds__(256, 1) fm_gemm_kernel(const GemmParams p) {
 }
 
 // ---- big tiles (many pairs per expert) -----------------------------------------------
-// Work-group: 256 pairs x 256 weight rows, 8 waves, two per SIMD. Wave w
-// computes pair half w >> 2 (128 pairs, 4 row blocks) against weight quarter
-// w & 3 (64 rows, 2 column blocks): the 128-pair tile's per-wave shape, with
-// each weight fragment now feeding 256 pairs and each pair fragment 256 rows,
-// so a stage moves 128 flop per byte into LDS (85 for the 128-pair tile), and
-// the second wave on each SIMD issues MFMAs while the first waits for its
-// fragment reads. K streams in 32-wide stages through a 4-deep ring (32 KiB
-// per stage: A 256 rows, then B 256 rows, of 64 bytes), in pairs: two stages
-// are in flight while the other two are read. Row r's 16-byte chunk c sits at
-// c ^ ((r >> 2) & 3):
-// 16 consecutive rows of one chunk (a fragment read's LDS cycle) then hit 16
-// distinct groups of 4 banks. Each wave moves A rows 32w..32w+31 and B rows
-// 32w..32w+31 of every stage (two 16-row LDS-DMA instructions each; A rows
-// past the tile's last pair are skipped).
+// Work-group: 256 pairs x 256 weight rows, 8 waves, two per SIMD. Wave w takes
+// the 32-pair row blocks of parity w >> 2 against weight quarter w & 3 (64
+// rows, 2 column blocks): 4 x 2 accumulator blocks when the tile is full. The
+// blocks alternate between the two wave halves, so a tile of n pairs costs
+// ceil(n / 64) block rows of MFMA time whatever n is.
+// K streams in 64-wide stages (128 bytes of each row: a 64-byte piece costs L2
+// and the vector cache as much as a whole 128-byte line, 17 against 31 TB/s
+// measured): the pairs' rows (A, from L2) through two LDS buffers of 32 KiB,
+// the weights (B, first touched by the launch, so from HBM) through three.
+// Row r's 16-byte chunk c sits at swz(r, c), as in the 128-pair tile. Wave w
+// moves the 8-row DMA groups w + 8 g of A and of B; groups of A past the
+// tile's last pair are skipped.
+// What bounds it: MFMA issue (a full tile is 32 x 2 MFMAs of 32 cycles per
+// SIMD and stage against 774 cycles of LDS reads) and the latency of the
+// weights, so the loop reads the fragments of a 16-wide k step between the
+// MFMAs of the one before, the stage barrier sits between two MFMA batches,
+// and the DMAs ride between MFMAs, two stages ahead for the weights.
+// Gate-up / down at K = 2048, N = 1024 (rocprof medians), against 32-wide
+// stages in pairs, the row blocks of one half per wave half and 2-byte stores:
+// M = 4096, E = 8, topk = 2 123 / 69 -> 83 / 46 us (825 TFLOP/s); M = 4001,
+// E = 64, topk = 6 317 / 176 -> 258 / 146 us. One full gate-up tile takes 2.6
+// us to its first stage and 48 us (two weight buffers) for its 32 stages, of
+// which the MFMAs are 31.
 constexpr int kBigRows = 256;                        // pairs per tile
-constexpr int kBigBK = 32;                           // k per stage
-constexpr int kBigStages = 4;
-constexpr int kBigRowBytes = kBigBK * 2;             // 64
-constexpr int kBigAStage = kBigRows * kBigRowBytes;  // 16 KiB
-constexpr int kBigStage = 2 * kBigAStage;            // A then B (256 weight rows)
+constexpr int kBigABufs = 2;
+constexpr int kBigBBufs = 3;
+constexpr int kBigPart = kBigRows * kRowBytes;       // one stage of A or B, 32 KiB
+constexpr int kBigLds = (kBigABufs + kBigBBufs) * kBigPart;  // 160 KiB
+// epilogue: each wave passes its outputs through LDS lines of its own
+constexpr int kBigPitchGated = 64 + 16;              // 32 outputs of a pair, padded
+constexpr int kBigPitchDown = 128 + 16;              // 64 outputs of a pair, padded
+constexpr int kBigPairs = 8 * 128 * kBigPitchDown;   // then the waves' pair ids (128 each)
 static_assert(kLargeCols == 256, "the big tile's weight rows are the large tile's");
+static_assert(kBigPairs + 8 * 128 * 4 <= kBigLds, "the epilogue fits");
 
-__device__ __forceinline__ int swz4(int row, int chunk) { return chunk ^ ((row >> 2) & 3); }
+// silu in fp32 with the hardware exponential and reciprocal: exp(-x) as
+// 2^(t + r), t + r = -x log2(e) to about 2^-48, within 2 ulp of the exact value.
+__device__ __forceinline__ float silu_fast(float x) {
+  const float t = x * -1.44269504f;
+  const float r = __builtin_fmaf(x, -1.92596299e-8f, __builtin_fmaf(x, -1.44269504f, -t));
+  float e = __builtin_amdgcn_exp2f(t);
+  // (past 2^126 and for x = +-inf, r may not be finite: e is 0 or huge there)
+  const bool in = __builtin_fabsf(t) < 126.f;
+  e = in ? __builtin_fmaf(e, r * 0.693147181f, e) : e;
+  const float d = 1.f + e;
+  float q = __builtin_amdgcn_rcpf(d);
+  q = in ? __builtin_fmaf(__builtin_fmaf(-d, q, 1.f), q, q) : q;  // one Newton step
+  return x * q;
+}
 
-// The K loop and epilogue of one wave's share of a big tile; NRB = the 32-pair
-// row blocks of the wave's half holding pairs (0: DMAs and barriers only).
+// Work item (pair tile, column tile) of a big-tile work-group. Work-group b
+// runs on XCD b % 8 (dispatch is round-robin over the XCDs, in order of b).
+// The items, pair tile by pair tile, are cut into 8 equal runs, one per XCD: a
+// pair tile's gathered rows and an expert's weight rows then go to one L2 (two
+// at a cut). The plan puts the tiles of at most 128 pairs last (tiles[1] = the
+// number before them) when the launch has at most two items per CU, and each
+// XCD takes its run of those after its run of the others, so that what starts
+// last is short. At M = 4096, E = 8, topk = 2 (32-40 tiles x 8) each XCD then
+// holds one expert's four full tiles. False: no item for this work-group.
+__device__ __forceinline__ bool big_item(const GemmParams& p, int& tile, int& ct) {
+  const int nt = p.tiles[0], nb = p.tiles[1];
+  const int x = int(blockIdx.x) % kXcds;
+  int s = int(blockIdx.x) / kXcds;
+  const int ib = nb * p.col_tiles, is = (nt - nb) * p.col_tiles;
+  const int b0 = x * ib / kXcds, bn = (x + 1) * ib / kXcds - b0;
+  int item;
+  if (s < bn) {
+    item = b0 + s;
+  } else {
+    s -= bn;
+    const int s0 = x * is / kXcds;
+    if (s >= (x + 1) * is / kXcds - s0) return false;
+    item = ib + s0 + s;
+  }
+  tile = item / p.col_tiles;
+  ct = item % p.col_tiles;
+  return true;
+}
+
+// The K loop and epilogue of one wave's share of a big tile; NRB = its 32-pair
+// row blocks holding pairs (0: DMAs and barriers only).
 template <bool kGated, int NRB>
-__device__ __forceinline__ void big_tile(const GemmParams& p, const uint8_t* s_buf,
-                                         const int* s_pair, const float* s_wt,
+__device__ __forceinline__ void big_tile(const GemmParams& p, uint8_t* s_buf,
                                          const uint8_t* abase, const uint8_t* wbase,
-                                         const uint32_t (&a_off)[2], const uint32_t (&b_off)[2],
+                                         const uint32_t (&a_off)[4], const uint32_t (&b_off)[4],
                                          uint32_t lds0, int na, int start, int rows, int ct) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ph = wave >> 2;  // pair half
+  const int ph = wave >> 2;  // parity of the wave's row blocks
   const int wq = wave & 3;   // weight quarter
   const int l32 = lane & 31;
   const int hi = lane >> 5;
-  const int nst = p.kin / kBigBK;
-  auto issue = [&](int st) {
-    const uint32_t sb = lds0 + uint32_t((st % kBigStages) * kBigStage);
-    const int64_t k0 = int64_t(st) * kBigRowBytes;
-#pragma unroll
-    for (int g = 0; g < 2; ++g)
-      if (g < na) lds_dma(abase + k0, a_off[g], sb + uint32_t((2 * wave + g) * 1024));
-#pragma unroll
-    for (int g = 0; g < 2; ++g)
-      lds_dma(wbase + k0, b_off[g], sb + uint32_t(kBigAStage + (2 * wave + g) * 1024));
+  const int nst = p.kin / kBK;
+  constexpr int kRB = NRB > 0 ? NRB : 1;
+  // DMAs of a stage: A groups 0..3 into A buffer `ab`, B groups 0..3 into B buffer `bb`
+  auto dma_a = [&](int st, int ab, int g) {
+    if (g < na)
+      lds_dma(abase + int64_t(st) * kRowBytes, a_off[g],
+              lds0 + uint32_t(ab * kBigPart + (wave + 8 * g) * 1024));
+  };
+  auto dma_b = [&](int st, int bb, int g) {
+    lds_dma(wbase + int64_t(st) * kRowBytes, b_off[g],
+            lds0 + uint32_t((kBigABufs + bb) * kBigPart + (wave + 8 * g) * 1024));
   };
 
-  f32x16 acc[NRB > 0 ? NRB : 1][2];
+  // the pairs of this lane's accumulator columns and their weights
+  int pair[kRB];
+  float wt[kRB];
+  if constexpr (!kGated && NRB > 0) {
 #pragma unroll
-  for (int rb = 0; rb < (NRB > 0 ? NRB : 1); ++rb)
+    for (int rb = 0; rb < NRB; ++rb) pair[rb] = p.sorted[start + min(64 * rb + 32 * ph + l32, rows - 1)];
+#pragma unroll
+    for (int rb = 0; rb < NRB; ++rb) wt[rb] = p.wts[pair[rb]];
+  }
+
+  f32x16 acc[kRB][2];
+#pragma unroll
+  for (int rb = 0; rb < kRB; ++rb)
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[rb][cb][i] = 0.f;
 
-  // Stages go in pairs: one wait and barrier per pair. Before pair (st,
-  // st + 1) only its own loads are in flight; after the barrier the next
-  // pair's are issued into the buffers of the pair every wave has just
-  // finished (one barrier per 64 k instead of per 32: 1-7 % faster).
-  static_assert(kBigStages == 4, "two pairs of stage buffers");
-  for (int st = 0; st < 2 && st < nst; ++st) issue(st);
-  // one stage's fragment reads (both k-steps) and MFMAs
-  auto reads = [&](int st, bf16x8 (&bf)[2][2], bf16x8 (&af)[2][NRB > 0 ? NRB : 1]) {
-    const uint8_t* sa = s_buf + (st % kBigStages) * kBigStage;
-    const uint8_t* sb = sa + kBigAStage;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int c = 2 * kk + hi;
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const int lr = 64 * wq + 32 * cb + l32;
-        bf[kk][cb] = *reinterpret_cast<const bf16x8*>(sb + lr * kBigRowBytes + swz4(lr, c) * 16);
-      }
-#pragma unroll
-      for (int rb = 0; rb < NRB; ++rb) {
-        const int r = 128 * ph + 32 * rb + l32;
-        af[kk][rb] = *reinterpret_cast<const bf16x8*>(sa + r * kBigRowBytes + swz4(r, c) * 16);
-      }
-    }
+  // fragment f of one 16-wide k step: the 2 weight blocks, then the row blocks
+  struct Frags {
+    bf16x8 b[2], a[kRB];
   };
-  auto mfmas = [&](const bf16x8 (&bf)[2][2], const bf16x8 (&af)[2][NRB > 0 ? NRB : 1]) {
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int rb = 0; rb < NRB; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][rb], bf[kk][cb],
-                                                                 acc[rb][cb], 0, 0, 0);
+  auto read1 = [&](const uint8_t* sa, const uint8_t* sb, int kk, int f, Frags& fr) {
+    const int pos = swz(l32, 2 * kk + hi) * 16;
+    if (f < 2)
+      fr.b[f] = *reinterpret_cast<const bf16x8*>(sb + (64 * wq + 32 * f + l32) * kRowBytes + pos);
+    else if (f - 2 < NRB)
+      fr.a[f - 2] =
+          *reinterpret_cast<const bf16x8*>(sa + (32 * ph + 64 * (f - 2) + l32) * kRowBytes + pos);
   };
-  // nst is even: validate() requires K % 256 == 0 and N % 128 == 0
-  for (int st = 0; st < nst; st += 2) {
-    wait_vmcnt(0);
-    lds_barrier();
-    for (int s2 = st + 2; s2 < st + 4 && s2 < nst; ++s2) issue(s2);
-    if constexpr (NRB > 0) {
-      // the pair in one body: the second stage's fragment reads fly under
-      // the first's MFMAs (1-4 % against a loop over single stages)
-      bf16x8 bf0[2][2], af0[2][NRB], bf1[2][2], af1[2][NRB];
-      reads(st, bf0, af0);
-      reads(st + 1, bf1, af1);
-      mfmas(bf0, af0);
-      mfmas(bf1, af1);
-    }
-  }
-
-  // epilogue: lane holds column l32 of each column block and pair rows
-  // 128 * ph + 32 * rb + 8 * a + 4 * hi + b in register 4 * a + b
-  if constexpr (NRB > 0) {
+  // The MFMAs of step (fr), with the reads of the next step (sa, sb, kk) into
+  // `nx` between them unless kk < 0; `after(i)` runs after MFMA pair i.
+  auto step = [&](const Frags& fr, const uint8_t* sa, const uint8_t* sb, int kk, Frags& nx,
+                  auto after) {
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb) {
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+      for (int cb = 0; cb < 2; ++cb)
+        acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr.b[cb], fr.a[rb], acc[rb][cb], 0, 0, 0);
+      // all reads within the first NRB - 1 pairs (or the only one)
+      constexpr int kSlots = NRB > 1 ? NRB - 1 : 1;
+      if (kk >= 0 && rb < kSlots) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int r = 128 * ph + 32 * rb + 8 * a + 4 * hi + b;
-          if (r >= rows) continue;
-          const int ri = 4 * a + b;
-          if (kGated) {
-            const float g = bf16r(silu(bf16r(acc[rb][0][ri])));
-            const float u = bf16r(acc[rb][1][ri]) * g;
-            const int j = ct * (kLargeCols / 2) + 32 * wq + l32;
-            p.out[int64_t(start + r) * p.out_stride + j] = static_cast<__bf16>(u);
-          } else {
-            const int pair = s_pair[r];
-            const float w = s_wt[r];
+        for (int f = rb * (NRB + 2) / kSlots; f < (rb + 1) * (NRB + 2) / kSlots; ++f)
+          read1(sa, sb, kk, f, nx);
+      }
+      after(rb);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto nothing = [](int) {};
+
+  // nst >= 2: validate() requires K % 256 == 0 and N % 128 == 0
 #pragma unroll
-            for (int cb = 0; cb < 2; ++cb) {
-              const int f = ct * kLargeCols + 64 * wq + 32 * cb + l32;
-              p.out[int64_t(pair) * p.out_stride + f] =
-                  static_cast<__bf16>(bf16r(acc[rb][cb][ri]) * w);
-            }
+  for (int g = 0; g < 4; ++g) dma_a(0, 0, g);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) dma_b(0, 0, g);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) dma_a(1, 1, g);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) dma_b(1, 1, g);
+  if (nst > 2) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) dma_b(2, 2, g);
+  }
+  wait_vmcnt(na + (nst > 2 ? 8 : 4));
+  lds_barrier();
+  const uint8_t* const sb0 = s_buf + kBigABufs * kBigPart;
+  Frags f0, f1;
+#pragma unroll
+  for (int f = 0; f < NRB + 2; ++f) read1(s_buf, sb0, 0, f, f0);
+  int bb = 0;  // st % 3
+  for (int st = 0; st < nst; ++st) {
+    const uint8_t* sa = s_buf + (st & 1) * kBigPart;
+    const uint8_t* sb = sb0 + bb * kBigPart;
+    const int nb = bb == kBigBBufs - 1 ? 0 : bb + 1;
+    step(f0, sa, sb, 1, f1, nothing);
+    step(f1, sa, sb, 2, f0, nothing);
+    step(f0, sa, sb, 3, f1, nothing);
+    // stage st + 1 has landed (only the weights of stage st + 2 still fly), then
+    // it has for every wave, and every wave has read stage st (the last pass
+    // reads a stale stage ahead, unused)
+    if (st + 2 < nst)
+      wait_vmcnt(4);
+    else
+      wait_vmcnt(0);
+    lds_barrier();
+    // the DMAs into stage st's buffers: A of stage st + 2, B of stage st + 3
+    const bool ma = st + 2 < nst, mb = st + 3 < nst;
+    auto dmas = [&](int rb) {
+#pragma unroll
+      for (int d = rb * 8 / kRB; d < (rb + 1) * 8 / kRB; ++d) {
+        if (d < 4) {
+          if (ma) dma_a(st + 2, st & 1, d);
+        } else {
+          if (mb) dma_b(st + 3, bb, d - 4);
+        }
+      }
+    };
+    if constexpr (NRB == 0) dmas(0);
+    step(f1, s_buf + ((st + 1) & 1) * kBigPart, sb0 + nb * kBigPart, 0, f0, dmas);
+    bb = nb;
+  }
+
+  // epilogue: the lane holds, for pair row 64 * rb + 32 * ph + l32, weight rows
+  // 8 * a + 4 * hi + i of each column block in register 4 * a + i. The outputs
+  // go through this wave's own LDS lines, so that global stores write 64
+  // (gated) or 128 contiguous bytes of a row by 16 bytes per lane: 2 us instead
+  // of 5 for 2-byte stores straight from the accumulators.
+  lds_barrier();  // every wave's reads are done
+  if constexpr (NRB > 0) {
+    constexpr int kPitch = kGated ? kBigPitchGated : kBigPitchDown;
+    constexpr int kOuts = kGated ? 32 : 64;        // outputs per pair row and wave
+    constexpr int kLanes = kOuts / 8;              // lanes per row of a 16-byte store
+    uint8_t* const sw = s_buf + wave * (128 * kBigPitchDown);
+    int* const sp = reinterpret_cast<int*>(s_buf + kBigPairs) + 128 * wave;
+#pragma unroll
+    for (int rb = 0; rb < NRB; ++rb) {
+      uint8_t* line = sw + (32 * rb + l32) * kPitch + 8 * hi;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        if constexpr (kGated) {
+          bf16x4 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float g = bf16r(silu_fast(bf16r(acc[rb][0][4 * a + i])));
+            o[i] = static_cast<__bf16>(bf16r(acc[rb][1][4 * a + i]) * g);
+          }
+          *reinterpret_cast<bf16x4*>(line + 16 * a) = o;
+        } else {
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) {
+            bf16x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              o[i] = static_cast<__bf16>(bf16r(acc[rb][cb][4 * a + i]) * wt[rb]);
+            *reinterpret_cast<bf16x4*>(line + 64 * cb + 16 * a) = o;
           }
         }
+      }
+      if constexpr (!kGated) sp[32 * rb + l32] = pair[rb];  // both halves: the same value
+    }
+    asm volatile("" ::: "memory");  // one wave: its LDS operations run in order
+    const int c = lane % kLanes;
+#pragma unroll
+    for (int i = 0; i < 32 * NRB / (64 / kLanes); ++i) {
+      const int lr = i * (64 / kLanes) + lane / kLanes;     // row within the wave's
+      const int r = 64 * (lr >> 5) + 32 * ph + (lr & 31);   // row of the tile
+      if (r >= rows) continue;
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(sw + lr * kPitch + 16 * c);
+      __bf16* dst;
+      if constexpr (kGated)
+        dst = p.out + int64_t(start + r) * p.out_stride + ct * (kLargeCols / 2) + 32 * wq;
+      else
+        dst = p.out + int64_t(sp[lr]) * p.out_stride + ct * kLargeCols + 64 * wq;
+      *reinterpret_cast<bf16x8*>(dst + 8 * c) = v;
     }
   }
 }
 
 template <bool kGated>
 __global__ void __launch_bounds__(512, 1) fm_gemm_big_kernel(const GemmParams p) {
-  __shared__ __attribute__((aligned(1024))) uint8_t s_buf[kBigStages * kBigStage];
-  __shared__ int s_pair[kBigRows];
-  __shared__ float s_wt[kBigRows];
+  __shared__ __attribute__((aligned(1024))) uint8_t s_buf[kBigLds];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int tile, ct;
-  if (!xcd_item(p, tile, ct)) return;
+  if (!big_item(p, tile, ct)) return;
   const int32_t* tl = p.tiles + 4 + 4 * tile;
   const int e = __builtin_amdgcn_readfirstlane(tl[0]);
   const int start = __builtin_amdgcn_readfirstlane(tl[1]);
   const int rows = __builtin_amdgcn_readfirstlane(tl[2]);
 
-  if (tid < kBigRows) {
-    const int r = tid < rows ? tid : 0;
-    const int pair = p.sorted[start + r];
-    s_pair[tid] = pair;
-    if (!kGated) s_wt[tid] = p.wts[pair];
-  }
-  __syncthreads();
-
   // Per-lane DMA sources: instruction g of this wave moves LDS rows
-  // 32 * wave + 16 * g + lane / 4, lane & 3 being the chunk position there.
-  const int sub = lane >> 2;
-  const int pos = lane & 3;
-  uint32_t a_off[2], b_off[2];
+  // 8 * (wave + 8 * g) + lane / 8, lane & 7 being the chunk position there.
+  const int sub = lane >> 3;
+  const int pos = lane & 7;
+  uint32_t a_off[4], b_off[4];
+  int64_t arow[4];
 #pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    const int r = 32 * wave + 16 * g + sub;
-    const int c = swz4(r, pos);  // the chunk whose swizzled position is `pos`
-    const int64_t arow =
-        kGated ? int64_t(s_pair[r] / p.topk) : int64_t(start + (r < rows ? r : 0));
-    a_off[g] = uint32_t(arow * p.a_stride * 2 + c * 16);
+  for (int g = 0; g < 4; ++g) {
+    const int r = 8 * (wave + 8 * g) + sub;
+    const int at = start + (r < rows ? r : 0);
+    arow[g] = kGated ? int64_t(p.sorted[at]) : int64_t(at);
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int r = 8 * (wave + 8 * g) + sub;
+    const int c = swz(r, pos);  // the chunk whose swizzled position is `pos`
+    if (kGated) arow[g] = uint32_t(arow[g]) / uint32_t(p.topk);
+    a_off[g] = uint32_t(arow[g] * p.a_stride * 2 + c * 16);
     // weight row of LDS row r: weight quarter r >> 6, column block (r >> 5) & 1
     int wrow;
     if (kGated)  // gate rows j, up rows N + j, j = ct * 128 + 32 * (r >> 6) + (r & 31)
@@ -921,17 +1055,16 @@ __global__ void __launch_bounds__(512, 1) fm_gemm_big_kernel(const GemmParams p)
     b_off[g] = uint32_t(int64_t(wrow) * p.kin * 2 + c * 16);
   }
   // A instructions of this wave that hold a pair
-  const int na = max(0, min(2, (rows - 32 * wave + 15) / 16));
+  const int na = max(0, min(4, (rows - 8 * wave + 63) / 64));
   const uint8_t* abase = reinterpret_cast<const uint8_t*>(p.a);
   const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.w + int64_t(e) * p.w_estride);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
       uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)s_buf)));
 
-  // 32-pair row blocks of this wave's half that hold pairs
-  const int nrb = max(0, min(4, (rows - 128 * (wave >> 2) + 31) / 32));
-#define FM_BIG(n)                                                                          \
-  big_tile<kGated, n>(p, s_buf, s_pair, s_wt, abase, wbase, a_off, b_off, lds0, na, start, \
-                      rows, ct)
+  // 32-pair row blocks 2 i + (wave >> 2) that hold pairs
+  const int nrb = max(0, min(4, (rows - 32 * (wave >> 2) + 63) / 64));
+#define FM_BIG(n) \
+  big_tile<kGated, n>(p, s_buf, abase, wbase, a_off, b_off, lds0, na, start, rows, ct)
   switch (nrb) {
     case 0: FM_BIG(0); break;
     case 1: FM_BIG(1); break;
@@ -1349,6 +1482,8 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   pp.P = pl.P;
   pp.E = int(a->E);
   pp.tile_rows = pl.tile_rows;
+  // big tiles with at most two gate-up items per CU: what starts last is short
+  pp.split_small = pl.big && pl.max_tiles * (a->N / (kLargeCols / 2)) <= 512;
   if (a->M <= kFusedRouteTokens) {  // one launch, reported as the plan's
     void* ka[] = {&rp, &pp};
     if (!run(FM_KERNEL_PLAN, fn(fm_route_plan_kernel), dim3(1), dim3(1024), ka)) return FM_EHIP;
@@ -1396,7 +1531,7 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
     g2.fsum_stride = a->s_out;
   }
   g1.ct_per_wg = g2.ct_per_wg = 1;
-  // (MI355X: 256 CUs, one large or big work-group each)
+  // (MI355X: 256 CUs, one large work-group each)
   const double pairs_per_expert = double(pl.P) / double(a->E);
   for (GemmParams* g : {&g1, &g2})
     g->xcd_grid = pl.large && pairs_per_expert < 2.0 * pl.tile_rows &&
@@ -1412,6 +1547,8 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
     }
   }
   auto grid_of = [&](const GemmParams& g) {
+    if (pl.big)  // big_item: each XCD has at most 1 / 8 of the items of each size, rounded up
+      return unsigned(kXcds * (pl.max_tiles * g.col_tiles / kXcds + 2));
     if (pl.large)  // xcd_item: each XCD has up to ceil(tiles / 4) x ceil(col_tiles / 2) items
       return unsigned(kXcds * ((pl.max_tiles + kXcdTileGroups - 1) / kXcdTileGroups) *
                       ((g.col_tiles + kXcdColGroups - 1) / kXcdColGroups));
