@@ -584,16 +584,16 @@ MOE_FUSED_ROUTE_TOKENS = 16  # kFusedRouteTokens in csrc/fused_moe_gfx950.hip
 
 def moe_gemm_kernel(M, N, E, topk, gated):
     """The GEMM kernel fused_moe launches for this shape with flags 0: the
-    tile choice of make_plan in csrc/fused_moe_gfx950.hip, restated for the
+    choice of choose_tiles in csrc/fused_moe_gfx950.hip, restated for the
     report (the profiles' kernel traces name the launched kernel)."""
     P = M * topk
     avg = P / E
     g = "true" if gated else "false"
-    if avg > 24.0:
-        fills = 128.0 <= avg < 208.0 or avg >= 360.0
-        big = fills and (P // 256) * (N // 128) >= 256
-        return f"fm_gemm_big_kernel<{g}>" if big else f"fm_gemm_kernel<{g}>"
-    pb = 4 if avg > 24.0 and N % 256 == 0 else 2 if avg > 12.0 else 1
+    one_round = min(E, P) * math.ceil((avg + 1.5 * math.sqrt(avg)) / 256) * (N // 32) <= 256
+    if avg > 24.0 or (one_round and avg >= 4.0) or (N <= 512 and avg > 6.0) or \
+            (N % 256 != 0 and avg > 8.0):
+        return f"fm_gemm_kernel<{g}>"
+    pb = 2 if avg > 12.0 else 1
     if N % 256 == 0:
         return f"fm_stream_kernel<{g}, {pb}>"
     return f"fm_skinny_kernel<{g}, {pb}>"

@@ -45,13 +45,13 @@ enum {
 enum {
   FM_FLAG_LARGE_TILES = 1u,  /* 128-pair tiles whatever the tokens per expert */
   FM_FLAG_SMALL_TILES = 2u,  /* 16-pair weight-streaming tiles */
-  FM_FLAG_BIG_TILES = 4u,    /* (ABI version 2) 256-pair tiles, 8 waves per work-group;
-                                by default once experts average 256 pairs */
+  FM_FLAG_BIG_TILES = 4u,    /* (ABI version 2) 256-pair tiles whatever the tokens per
+                                expert */
   FM_FLAG_ORDERED_SUM = 8u   /* (ABI version 4) the final sum over a token's experts
                                 always runs as its own launch (the ascending-expert
                                 running bf16 sum), never as the down GEMM's bf16
-                                atomic adds into the output (topk <= 2 with
-                                streamed tiles); the result is the same bits.
+                                atomic adds into the output (topk <= 2 with up to
+                                24 pairs per expert); the result is the same bits.
                                 Combines with one tile flag. */
 };
 
@@ -91,9 +91,9 @@ enum {
   FM_KERNEL_GATEUP = 2,  /* x = h . w1^T, u = up * silu(gate)        */
   FM_KERNEL_DOWN = 3,    /* y = u . w2^T, times the routing weight   */
   FM_KERNEL_REDUCE = 4,  /* ascending-expert bf16 sum per token; since
-                            version 3 not launched for topk <= 2 with
-                            streamed (decode) tiles: the down GEMM adds
-                            into out itself                          */
+                            version 3 not launched for topk <= 2 with up
+                            to 24 pairs per expert (decode): the down
+                            GEMM adds into out itself                */
   FM_KERNEL_COUNT = 5
 };
 

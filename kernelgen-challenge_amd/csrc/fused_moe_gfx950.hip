@@ -17,13 +17,14 @@
 //   in ascending expert order (the order of the final sum).
 // fm_plan_kernel    one work-group: pairs (t, slot) counted per expert and
 //   listed by expert, tiles of up to `tile_rows` pairs of one expert.
-// fm_gemm_kernel<gated>   (tokens per expert > ~24) a tile of 128 pairs x
-//   256 weight rows per work-group, K in 64-wide stages through a 3-stage
-//   LDS ring filled by LDS-DMA (1 KiB per wave instruction, XOR-swizzled so
-//   the MFMA fragment reads are free of bank conflicts), 32x32x16 bf16 MFMA,
-//   fp32 accumulation. gated: w1 rows j (gate) and N + j (up) sit in the
-//   same lane and register, so silu(gate) * up is formed in the epilogue.
-//   Otherwise (w2): the epilogue multiplies by the pair's routing weight.
+// fm_gemm_kernel<gated>   (prefill, and decode over few experts) a tile of up
+//   to 256 pairs x 256 weight rows (wide) or 64 (narrow) per work-group, K in
+//   64-wide stages through LDS rings filled by LDS-DMA (1 KiB per wave
+//   instruction, XOR-swizzled so the MFMA fragment reads are free of bank
+//   conflicts), 32x32x16 bf16 MFMA, fp32 accumulation. gated: w1 rows j (gate)
+//   and N + j (up) sit in the same lane and register, so silu(gate) * up is
+//   formed in the epilogue. Otherwise (w2): the epilogue multiplies by the
+//   pair's routing weight.
 // fm_skinny_kernel<gated, PB>  (few tokens per expert: decode) the weights
 //   are the streamed operand: each wave loads its 32 weight rows' MFMA
 //   fragments straight from HBM into registers (8 k-steps, 24-32 KiB, in
@@ -32,7 +33,7 @@
 //   through LDS. 16x16x32 bf16 MFMA.
 // fm_reduce_kernel  out[t] = bf16 running sum of the token's topk weighted
 //   expert outputs, ascending expert order. Not launched when topk <= 2 and
-//   the tiles are streamed (decode): the routing launch clears out, and the
+//   experts have few pairs (decode): the routing launch clears out, and the
 //   down GEMM adds each weighted row into it with packed bf16 atomics (the
 //   two-term bf16 sum does not depend on the order).
 #include <hip/hip_ext.h>
@@ -40,6 +41,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "fused_moe.h"
@@ -58,52 +60,88 @@ constexpr int kMaxTopk = 32;
 // ---------------------------------------------------------------------------
 // workspace plan (host)
 // ---------------------------------------------------------------------------
-constexpr int kLargeRows = 128;   // pairs per tile of fm_gemm_kernel
-constexpr int kLargeCols = 256;   // weight rows per tile of fm_gemm_kernel
+constexpr int kTileRows = 256;    // pairs per tile of fm_gemm_kernel at most
+constexpr int kTileCols = 256;    // weight rows per wide tile
+constexpr int kNarrowCols = 64;   // weight rows per narrow tile
 constexpr int kBK = 64;           // k per LDS stage
-constexpr int kStages = 3;
+constexpr int kRowBytes = kBK * 2;
+constexpr int kCus = 256;         // MI355X
+constexpr int kXcds = 8;
 
 struct Plan {
   int64_t P;            // pairs = M * topk
+  int64_t nonempty;     // experts with a pair, at most
+  bool gemm;            // fm_gemm_kernel (else fm_stream_kernel or fm_skinny_kernel)
   int tile_rows;        // pairs per tile
-  bool large;           // fm_gemm_kernel (else fm_skinny_kernel)
-  bool big;             // large, with 256-pair tiles: fm_gemm_big_kernel
-  int pb;               // small tiles: 16-pair blocks per tile (1, 2 or 4)
+  int narrow_rows;      // gemm: tiles of at most this many pairs run as narrow ones
+  int pb;               // not gemm: 16-pair blocks per tile (1, 2 or 4)
   int64_t max_tiles;    // upper bound on sum_e ceil(count_e / tile_rows)
   size_t ids_off, wts_off, eoff_off, sorted_off, tiles_off, inter_off, y_off, bytes;
 };
 
 inline size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// The kernel and its tiles, from the average pairs per expert n (an expert's
+// count spreads about sqrt(n) around it) and the launch's work items per CU.
+// fm_gemm_kernel runs one work-group per CU, so what counts is how many rounds
+// of items there are and how long one is. Measured whole calls (us), wide 256 /
+// wide 128 / narrow, the chosen one in brackets:
+//   K = 2048, N = 1024, E = 8, topk = 2: M = 256 57 / 56 / [39], M = 512
+//   65 / 63 / [45], M = 700 74 / 61 / [51], M = 1024 89 / [65] / 87, M = 2048
+//   [93] / 109 / 123, M = 3000 [104] / 122 / 162;
+//   E = 64, topk = 6: M = 512 [198] / 198 / 211, M = 1024 [219] / 218 / 248;
+//   K = 4096, N = 2048, E = 8, topk = 2, M = 700: 147 / [132] / 166.
+//   Short last tiles narrow against wide: M = 4096, E = 8 [134] / 175; M =
+//   1500, K = 2048, N = 1408, E = 16, topk = 4 169 / [164]; M = 4001, E = 64,
+//   topk = 6 481 / [385].
+// The streamed tiles read each weight once into one short-lived work-group and
+// win where the weights of many experts are the traffic (E = 64, M = 64: 163
+// against 183; M = 8: 108 against 122) and below 4 pairs per expert; with at
+// most one narrow item per CU fm_gemm_kernel wins from there (E = 8, M = 16: 35
+// against 38; M = 64: 36 against 41), and from 6 or 8 pairs where the streamed
+// kernel's own pipelines are short or absent (N <= 512: E = 128, M = 100, topk
+// = 8 93 against 107; N not a multiple of 256: E = 16, M = 60, topk = 4,
+// N = 1408 79 against 90).
+void choose_tiles(const fm_args* a, Plan& p) {
+  const double n = double(p.P) / double(a->E), sd = sqrt(n);
+  auto tiles = [&](double pairs, int rows) { return double(p.nonempty) * ceil(pairs / rows); };
+  const double cols = double(a->N) / (kTileCols / 2), narrow = double(a->N) / (kNarrowCols / 2);
+  const bool one_round = tiles(n + 1.5 * sd, kTileRows) * narrow <= kCus;
+  p.tile_rows = kTileRows;
+  p.narrow_rows = 0;
+  if (a->flags & (FM_FLAG_LARGE_TILES | FM_FLAG_BIG_TILES))
+    p.gemm = true;
+  else if (a->flags & FM_FLAG_SMALL_TILES)
+    p.gemm = false;
+  else
+    p.gemm = n > 24.0 || (one_round && n >= 4.0) || (a->N <= 512 && n > 6.0) ||
+             (a->N % 256 != 0 && n > 8.0);
+  // 16 or 32 pairs per small tile (64 only when forced)
+  p.pb = n > 24.0 && a->N % 256 == 0 ? 4 : n > 12.0 ? 2 : 1;
+  if (!p.gemm) {
+    p.tile_rows = 16 * p.pb;
+  } else if (a->flags & FM_FLAG_LARGE_TILES) {
+    p.tile_rows = 128;
+  } else if (one_round && (a->flags & FM_FLAG_BIG_TILES) == 0) {
+    p.narrow_rows = kTileRows;
+  } else if (tiles(n + 0.5 * sd, 128) * cols <= kCus && (a->flags & FM_FLAG_BIG_TILES) == 0) {
+    p.tile_rows = 128;
+  } else {
+    // an expert's last tile goes narrow when it has at most 128 pairs, if that
+    // saves a round of wide items and is itself at most two rounds
+    const double wide = double(p.nonempty) * floor((n + sd + 127.0) / kTileRows) * cols;
+    if (ceil(tiles(n + sd, kTileRows) * cols / kCus) > ceil(wide / kCus) &&
+        double(p.nonempty) * narrow <= 2 * kCus)
+      p.narrow_rows = 128;
+  }
+}
+
 Plan make_plan(const fm_args* a) {
   Plan p{};
   p.P = a->M * a->topk;
-  const double avg = double(p.P) / double(a->E);  // pairs per expert on average
-  if (a->flags & (FM_FLAG_LARGE_TILES | FM_FLAG_BIG_TILES))
-    p.large = true;
-  else if (a->flags & FM_FLAG_SMALL_TILES)
-    p.large = false;
-  else
-    p.large = avg > 24.0;
-  // 256-pair tiles when an expert's pairs fill them well and their gate-up
-  // GEMM still has a work-group for each of MI355X's 256 CUs (P / 256 pair
-  // tiles x N / 128 column tiles; fewer, and the 128-pair tiles' larger grid
-  // is faster: measured at M = 1024, 2048 with E = 8). Which fills better
-  // depends on the pairs per expert (K = 2048, N = 1024, E = 64, whole
-  // calls): 256-pair tiles win at 136-192 on average (most experts fit one,
-  // 4-8 %) and from 384 on; 128-pair tiles below 130 and at 225-336, where
-  // many experts spill a few pairs into a second, nearly empty 256-pair tile
-  // (2-10 %).
-  const bool fills = (avg >= 128.0 && avg < 208.0) || avg >= 360.0;
-  p.big = (a->flags & FM_FLAG_BIG_TILES) != 0 ||
-          ((a->flags & FM_FLAG_LARGE_TILES) == 0 && p.large && fills &&
-           (p.P / 256) * (a->N / 128) >= 256);
-  // 16 or 32 pairs per small tile (64 only when forced; measured slower than
-  // the large tiles at 48 pairs per expert)
-  p.pb = avg > 24.0 && a->N % 256 == 0 ? 4 : avg > 12.0 ? 2 : 1;
-  p.tile_rows = p.big ? 256 : p.large ? kLargeRows : 16 * p.pb;
-  const int64_t nonempty = a->E < p.P ? a->E : p.P;
-  p.max_tiles = p.P / p.tile_rows + nonempty;
+  p.nonempty = a->E < p.P ? a->E : p.P;
+  choose_tiles(a, p);
+  p.max_tiles = p.P / p.tile_rows + p.nonempty;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -126,7 +164,7 @@ int validate(const fm_args* a) {
   if (a->M < 0 || a->K <= 0 || a->N <= 0 || a->E <= 0 || a->topk <= 0) return FM_EINVAL;
   if (a->topk > a->E) return FM_EINVAL;
   if (a->E > kMaxExperts || a->topk > kMaxTopk) return FM_EUNSUPPORTED;
-  if (a->K % kLargeCols != 0 || a->N % (kLargeCols / 2) != 0) return FM_EUNSUPPORTED;
+  if (a->K % kTileCols != 0 || a->N % (kTileCols / 2) != 0) return FM_EUNSUPPORTED;
   const uint32_t tile_flags = a->flags & (FM_FLAG_LARGE_TILES | FM_FLAG_SMALL_TILES |
                                           FM_FLAG_BIG_TILES);
   if ((a->flags & ~(tile_flags | FM_FLAG_ORDERED_SUM)) != 0 ||
@@ -348,11 +386,11 @@ struct PlanParams {
   const int32_t* ids;
   int32_t* eoff;      // [E + 1] first sorted position of each expert
   int32_t* sorted;    // [P] pair ids (t * topk + slot) grouped by expert
-  int32_t* tiles;     // [0] = tile count, [1] = tiles before the small ones (of all
-                      // with split_small = 0), then int4 (expert, start, rows, 0) per tile
+  int32_t* tiles;     // [0] = tile count, [1] = tiles before the narrow ones, then
+                      // int4 (expert, start, rows, 0) per tile
   int64_t P;
   int E, tile_rows;
-  int split_small;    // list the tiles of at most tile_rows / 2 pairs last
+  int narrow_rows;    // tiles of at most this many pairs are listed last (narrow tiles)
 };
 
 struct PlanSmem {
@@ -369,9 +407,15 @@ __device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
   int* s_off = sm.off;
   int* s_toff = sm.toff;
   int* s_soff = sm.soff;
-  // an expert's last tile goes into the list of small ones
-  auto small_tile = [&](int n) {
-    return p.split_small && n % p.tile_rows > 0 && n % p.tile_rows <= p.tile_rows / 2;
+  // tiles of an expert with n pairs, and how many of them (the last one, or
+  // all) are narrow
+  // (tile_rows is a power of two)
+  const int log_rows = __builtin_ctz(p.tile_rows);
+  auto tiles_of = [&](int n) { return (n + p.tile_rows - 1) >> log_rows; };
+  auto narrow_of = [&](int n) {
+    const int nt = tiles_of(n);
+    return p.tile_rows <= p.narrow_rows ? nt
+                                        : n > 0 && n - (nt - 1) * p.tile_rows <= p.narrow_rows;
   };
   int* s_cur = sm.cur;
   const int tid = threadIdx.x;
@@ -387,18 +431,23 @@ __device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
     for (int c = 0; c < kMaxExperts / 64; ++c) {
       const int e = 64 * c + tid;
       const int v = e < p.E ? s_cnt[e] : 0;
-      const int sv = small_tile(v) ? 1 : 0;
-      const int tv = (v + p.tile_rows - 1) / p.tile_rows - sv;
+      const int sv = narrow_of(v);
+      const int tv = tiles_of(v) - sv;
       int incl = v, tincl = tv, sincl = sv;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int a = __shfl_up(incl, o);
         const int b = __shfl_up(tincl, o);
-        const int d = __shfl_up(sincl, o);
         if (tid >= o) {
           incl += a;
           tincl += b;
-          sincl += d;
+        }
+      }
+      if (p.narrow_rows > 0) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int d = __shfl_up(sincl, o);
+          if (tid >= o) sincl += d;
         }
       }
       if (e < p.E) {
@@ -429,8 +478,8 @@ __device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
   for (int e = tid; e < p.E; e += 1024) {
     const int n = s_cnt[e];
     for (int k = 0; k * p.tile_rows < n; ++k) {
-      const bool last = (k + 1) * p.tile_rows >= n;
-      const int at = last && small_tile(n) ? s_toff[p.E] + s_soff[e] : s_toff[e] + k;
+      const int wide = tiles_of(n) - narrow_of(n);
+      const int at = k < wide ? s_toff[e] + k : s_toff[p.E] + s_soff[e] + k - wide;
       int32_t* tl = p.tiles + 4 + 4 * at;
       tl[0] = e;
       tl[1] = s_off[e] + k * p.tile_rows;
@@ -498,10 +547,10 @@ struct GemmParams {
   int nout;              // GEMM 1: N (gate rows; up rows follow); GEMM 2: K
   int topk;
   int col_tiles;         // output-column tiles per pair tile
+  int narrow_cols;       // ... of a narrow tile (fm_gemm_kernel)
   int ct_per_wg;         // column tiles one work-group runs (fm_stream_kernel)
-  int xcd_grid;          // large tiles: the 2 x 4 XCD grid of xcd_item
-  // GEMM 2 with topk <= 2 (fm_stream_kernel): add each pair's bf16 row into
-  // the token's output row instead of writing yw (null: write yw)
+  // GEMM 2 with topk <= 2 (decode): add each pair's bf16 row into the token's
+  // output row instead of writing yw (null: write yw)
   __bf16* fsum;
   int64_t fsum_stride;
 };
@@ -517,270 +566,74 @@ __device__ __forceinline__ void add_bf16x2(__bf16* out, __bf16 a0, __bf16 a1) {
   asm volatile("global_atomic_pk_add_bf16 %0, %1, off sc1" : : "v"(out), "v"(v) : "memory");
 }
 
-// Work item (pair tile, column tile) of a large GEMM work-group. Work-group b
-// runs on XCD b % 8 (dispatch is round-robin over the XCDs, in order of b).
-// Plainly, b -> (b / col_tiles, b % col_tiles): column tile c of every pair
-// tile runs on XCD c % 8, so a weight tile is read into one L2 and shared
-// there by the pair tiles of its expert, while every pair tile's gathered A
-// rows are read into col_tiles L2s. With p.xcd_grid the XCDs form a 2 x 4 grid
-// instead: XCD x takes the column tiles of half x % 2 of every pair tile in
-// its contiguous quarter x / 2 of the tile table, pair tile by pair tile, so a
-// pair tile's A rows go to two L2s, and an expert's pair tiles (adjacent in
-// the table) still share its weight rows in one L2. The host sets xcd_grid
-// when experts average fewer than two pair tiles and the items outnumber the
-// CUs (1-7 % faster at M = 512-3072, E = 64, topk = 6, K = 2048, N = 1024).
-// False: no item for this work-group.
-constexpr int kXcds = 8;
-constexpr int kXcdColGroups = 2;
-constexpr int kXcdTileGroups = kXcds / kXcdColGroups;
-
-__device__ __forceinline__ bool xcd_item(const GemmParams& p, int& tile, int& ct) {
-  const int nt = p.tiles[0];
-  const int b = int(blockIdx.x);
-  if (!p.xcd_grid) {
-    tile = b / p.col_tiles;
-    ct = b % p.col_tiles;
-    return tile < nt;
-  }
-  const int x = b % kXcds, s = b / kXcds;
-  const int cg = x % kXcdColGroups, tg = x / kXcdColGroups;
-  const int c0 = cg * p.col_tiles / kXcdColGroups;
-  const int cn = (cg + 1) * p.col_tiles / kXcdColGroups - c0;
-  const int t0 = tg * nt / kXcdTileGroups;
-  const int tn = (tg + 1) * nt / kXcdTileGroups - t0;
-  if (cn <= 0 || s >= tn * cn) return false;
-  tile = t0 + s / cn;
-  ct = c0 + s % cn;
-  return true;
-}
-
-// ---- large tiles -------------------------------------------------------------
-// LDS stage: A 128 rows x 128 B, then B 256 rows x 128 B. Row r's 16-byte
-// chunk c (k = 8c..8c+7 of the stage) sits at chunk position c ^ ((r >> 1) & 7):
-// a 32x32x16 fragment read (lanes 0..15 = 16 consecutive rows, one chunk)
-// then covers all 64 banks once. An LDS-DMA instruction writes 8 rows
-// (1 KiB) lane-linearly, so each lane loads the global chunk that belongs at
-// its position.
-constexpr int kRowBytes = kBK * 2;                  // 128
-constexpr int kAStage = kLargeRows * kRowBytes;     // 16 KiB
-constexpr int kBStage = kLargeCols * kRowBytes;     // 32 KiB
-constexpr int kStage = kAStage + kBStage;           // 48 KiB
-
-__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
-
-// The K loop and epilogue of one tile with NRB row blocks (of 32 pairs)
-// holding pairs: full tiles run NRB = 4, an expert's last tile fewer.
-template <bool kGated, int NRB>
-__device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* s_buf, const int* s_pair,
-                                          const float* s_wt, const uint8_t* abase,
-                                          const uint8_t* wbase, const uint32_t (&a_off)[4],
-                                          const uint32_t (&b_off)[8], uint32_t lds0, int start,
-                                          int rows, int ct) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31;
-  const int hi = lane >> 5;
-  const int nst = p.kin / kBK;
-  // A instructions of this wave that hold a pair (rows 32 * wave + 8 * g ..):
-  // the rows past the tile's last pair are never loaded (nor read)
-  const int na = max(0, min(4, (rows - 32 * wave + 7) / 8));
-  // DMA d (0..11) of a stage: A instruction d (d < 4), else B instruction d - 4
-  auto dma = [&](int st, int d) {
-    const uint32_t sb = lds0 + uint32_t((st % kStages) * kStage);
-    if (d < 4) {
-      if (d < na)
-        lds_dma(abase + int64_t(st) * kRowBytes, a_off[d], sb + uint32_t((4 * wave + d) * 1024));
-    } else {
-      lds_dma(wbase + int64_t(st) * kRowBytes, b_off[d - 4],
-              sb + uint32_t(kAStage + (8 * wave + d - 4) * 1024));
-    }
-  };
-  auto issue = [&](int st) {
-#pragma unroll
-    for (int d = 0; d < 12; ++d) dma(st, d);
-  };
-
-  f32x16 acc[NRB][2];
-#pragma unroll
-  for (int rb = 0; rb < NRB; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[rb][cb][i] = 0.f;
-
-  issue(0);
-  if (nst > 1) issue(1);
-  for (int st = 0; st < nst; ++st) {
-    // this wave's loads of stage st are complete (na + 8 per stage; the
-    // ones of stage st + 1 may still fly), then every wave's are
-    wait_vmcnt(st + 1 < nst ? na + 8 : 0);
-    lds_barrier();
-    // stage st + 2 goes into the buffer every wave finished reading; its 12
-    // DMAs are spread over this stage's MFMAs (one per 2 MFMAs at NRB = 4)
-    const bool more = st + 2 < nst;
-    const uint8_t* sa = s_buf + (st % kStages) * kStage;
-    const uint8_t* sb = sa + kAStage;
-#pragma unroll
-    for (int kk = 0; kk < kBK / 16; ++kk) {
-      const int c = 2 * kk + hi;
-      bf16x8 bf[2];
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const int lr = 64 * wave + 32 * cb + l32;
-        bf[cb] = *reinterpret_cast<const bf16x8*>(sb + lr * kRowBytes + swz(lr, c) * 16);
-      }
-#pragma unroll
-      for (int rb = 0; rb < NRB; ++rb) {
-        const int r = 32 * rb + l32;
-        const bf16x8 af = *reinterpret_cast<const bf16x8*>(sa + r * kRowBytes + swz(r, c) * 16);
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf[cb], acc[rb][cb], 0, 0, 0);
-        constexpr int kSlots = 4 * NRB;  // MFMA pairs per stage
-        const int slot = kk * NRB + rb;
-        if (more) {
-#pragma unroll
-          for (int d = (slot * 12) / kSlots; d < ((slot + 1) * 12) / kSlots; ++d) dma(st + 2, d);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // keep the DMAs between the MFMAs
-      }
-    }
-  }
-
-  // epilogue: lane holds column l32 of each column block and pair rows
-  // 32 * rb + 8 * a + 4 * hi + b in register 4 * a + b
-#pragma unroll
-  for (int rb = 0; rb < NRB; ++rb) {
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int r = 32 * rb + 8 * a + 4 * hi + b;
-        if (r >= rows) continue;
-        const int ri = 4 * a + b;
-        if (kGated) {
-          const float g = bf16r(silu(bf16r(acc[rb][0][ri])));
-          const float u = bf16r(acc[rb][1][ri]) * g;
-          const int j = ct * (kLargeCols / 2) + 32 * wave + l32;
-          p.out[int64_t(start + r) * p.out_stride + j] = static_cast<__bf16>(u);
-        } else {
-          const int pair = s_pair[r];
-          const float w = s_wt[r];
-#pragma unroll
-          for (int cb = 0; cb < 2; ++cb) {
-            const int f = ct * kLargeCols + 64 * wave + 32 * cb + l32;
-            p.out[int64_t(pair) * p.out_stride + f] =
-                static_cast<__bf16>(bf16r(acc[rb][cb][ri]) * w);
-          }
-        }
-      }
-  }
-}
-
-template <bool kGated>
-__global__ void __launch_bounds__(256, 1) fm_gemm_kernel(const GemmParams p) {
-  __shared__ __attribute__((aligned(1024))) uint8_t s_buf[kStages * kStage];
-  __shared__ int s_pair[kLargeRows];
-  __shared__ float s_wt[kLargeRows];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-  int tile, ct;
-  if (!xcd_item(p, tile, ct)) return;
-  const int32_t* tl = p.tiles + 4 + 4 * tile;
-  const int e = __builtin_amdgcn_readfirstlane(tl[0]);
-  const int start = __builtin_amdgcn_readfirstlane(tl[1]);
-  const int rows = __builtin_amdgcn_readfirstlane(tl[2]);
-
-  if (tid < kLargeRows) {
-    const int r = tid < rows ? tid : 0;
-    const int pair = p.sorted[start + r];
-    s_pair[tid] = pair;
-    if (!kGated) s_wt[tid] = p.wts[pair];
-  }
-  __syncthreads();
-
-  // Per-lane DMA sources. A: this wave's 4 instructions cover tile rows
-  // 32 * wave + 8 * g + lane / 8; B: its 8 instructions cover its own 64
-  // weight rows (LDS rows 64 * wave + 8 * g + lane / 8).
-  const int sub = lane >> 3;       // row within the instruction's 8
-  const int pos = lane & 7;        // chunk position within the row
-  uint32_t a_off[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int r = 32 * wave + 8 * g + sub;
-    const int c = swz(r, pos);  // the chunk whose swizzled position is `pos`
-    const int64_t arow = kGated ? int64_t(s_pair[r] / p.topk) : int64_t(start + (r < rows ? r : 0));
-    a_off[g] = uint32_t(arow * p.a_stride * 2 + c * 16);
-  }
-  uint32_t b_off[8];
-#pragma unroll
-  for (int g = 0; g < 8; ++g) {
-    const int lr = 64 * wave + 8 * g + sub;   // LDS row of the B stage
-    const int cb = (lr >> 5) & 1;             // column block of the wave
-    const int i = lr & 31;
-    int wrow;
-    if (kGated)  // gate rows j, up rows N + j, j = ct * 128 + 32 * wave + i
-      wrow = (cb ? p.nout : 0) + ct * (kLargeCols / 2) + 32 * wave + i;
-    else         // features f = ct * 256 + lr
-      wrow = ct * kLargeCols + lr;
-    b_off[g] = uint32_t(int64_t(wrow) * p.kin * 2 + swz(lr, pos) * 16);
-  }
-  const uint8_t* abase = reinterpret_cast<const uint8_t*>(p.a);
-  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.w + int64_t(e) * p.w_estride);
-  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
-      uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)s_buf)));
-
-  const int nrb = (rows + 31) / 32;  // 32-pair row blocks holding pairs
-#define FM_TILE(n) \
-  gemm_tile<kGated, n>(p, s_buf, s_pair, s_wt, abase, wbase, a_off, b_off, lds0, start, rows, ct)
-  switch (nrb) {
-    case 1: FM_TILE(1); break;
-    case 2: FM_TILE(2); break;
-    case 3: FM_TILE(3); break;
-    default: FM_TILE(4); break;
-  }
-#undef FM_TILE
-}
-
-// ---- big tiles (many pairs per expert) -----------------------------------------------
-// Work-group: 256 pairs x 256 weight rows, 8 waves, two per SIMD. Wave w takes
-// the 32-pair row blocks of parity w >> 2 against weight quarter w & 3 (64
-// rows, 2 column blocks): 4 x 2 accumulator blocks when the tile is full. The
-// blocks alternate between the two wave halves, so a tile of n pairs costs
-// ceil(n / 64) block rows of MFMA time whatever n is.
+// ---- fm_gemm_kernel ----------------------------------------------------------------
+// Work-group of a wide tile: 256 pairs x 256 weight rows, 8 waves, two per
+// SIMD. Wave w takes the 32-pair row blocks of parity w >> 2 against weight
+// quarter w & 3 (64 rows, 2 column blocks): 4 x 2 accumulator blocks when the
+// tile is full. The blocks alternate between the two wave halves, so a tile of
+// n pairs costs ceil(n / 64) block rows of MFMA time whatever n is. A narrow
+// tile has 64 weight rows and wave w takes row block w: four times the
+// work-groups, each with a short stage (24 or 40 KiB) and so six or four of
+// them in LDS. They fill the chip where wide tiles are too few, and run an
+// expert's short last tile in a third of the time (8 against 20 us).
 // K streams in 64-wide stages (128 bytes of each row: a 64-byte piece costs L2
 // and the vector cache as much as a whole 128-byte line, 17 against 31 TB/s
 // measured): the pairs' rows (A, from L2) through two LDS buffers of 32 KiB,
 // the weights (B, first touched by the launch, so from HBM) through three.
-// Row r's 16-byte chunk c sits at swz(r, c), as in the 128-pair tile. Wave w
-// moves the 8-row DMA groups w + 8 g of A and of B; groups of A past the
-// tile's last pair are skipped.
+// Row r's 16-byte chunk c sits at swz(r, c): a 32x32x16 fragment read (lanes
+// 0..15 = 16 consecutive rows, one chunk) then covers all 64 banks once; each
+// lane of an LDS-DMA loads the chunk that belongs at its position. Wave w moves
+// the 8-row DMA groups w + 8 g of A and of B; groups of A past the tile's last
+// pair are skipped. Every form runs the same MFMA sequence per output element,
+// so they agree bit for bit.
 // What bounds it: MFMA issue (a full tile is 32 x 2 MFMAs of 32 cycles per
 // SIMD and stage against 774 cycles of LDS reads) and the latency of the
 // weights, so the loop reads the fragments of a 16-wide k step between the
 // MFMAs of the one before, the stage barrier sits between two MFMA batches,
 // and the DMAs ride between MFMAs, two stages ahead for the weights.
 // Gate-up / down at K = 2048, N = 1024 (rocprof medians), against 32-wide
-// stages in pairs, the row blocks of one half per wave half and 2-byte stores:
-// M = 4096, E = 8, topk = 2 123 / 69 -> 83 / 46 us (825 TFLOP/s); M = 4001,
-// E = 64, topk = 6 317 / 176 -> 258 / 146 us. One full gate-up tile takes 2.6
-// us to its first stage and 48 us (two weight buffers) for its 32 stages, of
-// which the MFMAs are 31.
-constexpr int kBigRows = 256;                        // pairs per tile
-constexpr int kBigABufs = 2;
-constexpr int kBigBBufs = 3;
-constexpr int kBigPart = kBigRows * kRowBytes;       // one stage of A or B, 32 KiB
-constexpr int kBigLds = (kBigABufs + kBigBBufs) * kBigPart;  // 160 KiB
+// stages in pairs, the row blocks of one half per wave half, 2-byte stores and
+// wide tiles only: M = 4096, E = 8, topk = 2 123 / 69 -> 78 / 44 us; M = 4001,
+// E = 64, topk = 6 317 / 176 -> 258 / 146 us. A full wide gate-up tile takes
+// 2.9 us to its first stage, 49 us for its 32 stages (1.40 PFLOP/s over 256
+// CUs; without its loads 41 us) and 3.9 us for its epilogue.
+enum TileForm { kWide, kNarrow128, kNarrow256 };  // narrow: up to 128 or 256 pairs
+
+__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
+
+template <TileForm kForm>
+struct TileShape {  // wide
+  static constexpr int kWq = 4;                 // 64-row weight parts, one per wave
+  static constexpr int kRows = kTileRows;       // pairs
+  static constexpr int kABufs = 2, kBBufs = 3;  // stages of A and B in LDS
+};
+template <>
+struct TileShape<kNarrow128> {
+  static constexpr int kWq = 1, kRows = 128, kABufs = 6, kBBufs = 6;
+};
+template <>
+struct TileShape<kNarrow256> {
+  static constexpr int kWq = 1, kRows = 256, kABufs = 4, kBBufs = 4;
+};
+template <TileForm kForm>
+struct TileLds : TileShape<kForm> {
+  using S = TileShape<kForm>;
+  static constexpr int kPh = 8 / S::kWq;             // waves that share a weight part
+  static constexpr int kCols = 64 * S::kWq;          // weight rows
+  static constexpr int kA = S::kRows * kRowBytes;    // bytes of one stage of A, of B
+  static constexpr int kB = kCols * kRowBytes;
+  static constexpr int kBytes = S::kABufs * kA + S::kBBufs * kB;
+  static constexpr int kAGroups = S::kRows / 64;     // DMA groups per wave and stage
+  static constexpr int kBGroups = kCols / 64;
+};
+constexpr int kGemmLds = TileLds<kWide>::kBytes;  // 160 KiB
+static_assert(TileLds<kNarrow128>::kBytes <= kGemmLds && TileLds<kNarrow256>::kBytes <= kGemmLds,
+              "narrow stages fit");
 // epilogue: each wave passes its outputs through LDS lines of its own
-constexpr int kBigPitchGated = 64 + 16;              // 32 outputs of a pair, padded
-constexpr int kBigPitchDown = 128 + 16;              // 64 outputs of a pair, padded
-constexpr int kBigPairs = 8 * 128 * kBigPitchDown;   // then the waves' pair ids (128 each)
-static_assert(kLargeCols == 256, "the big tile's weight rows are the large tile's");
-static_assert(kBigPairs + 8 * 128 * 4 <= kBigLds, "the epilogue fits");
+constexpr int kPitchGated = 64 + 16;              // 32 outputs of a pair, padded
+constexpr int kPitchDown = 128 + 16;              // 64 outputs of a pair, padded
+constexpr int kPairsOff = 8 * 128 * kPitchDown;   // then the waves' pair ids (128 each)
+static_assert(kPairsOff + 8 * 128 * 4 <= kGemmLds, "the epilogue fits");
 
 // silu in fp32 with the hardware exponential and reciprocal: exp(-x) as
 // 2^(t + r), t + r = -x log2(e) to about 2^-48, within 2 ulp of the exact value.
@@ -797,60 +650,98 @@ __device__ __forceinline__ float silu_fast(float x) {
   return x * q;
 }
 
-// Work item (pair tile, column tile) of a big-tile work-group. Work-group b
+// Work item (pair tile, column tile) of a work-group. Work-group b
 // runs on XCD b % 8 (dispatch is round-robin over the XCDs, in order of b).
 // The items, pair tile by pair tile, are cut into 8 equal runs, one per XCD: a
 // pair tile's gathered rows and an expert's weight rows then go to one L2 (two
-// at a cut). The plan puts the tiles of at most 128 pairs last (tiles[1] = the
-// number before them) when the launch has at most two items per CU, and each
-// XCD takes its run of those after its run of the others, so that what starts
-// last is short. At M = 4096, E = 8, topk = 2 (32-40 tiles x 8) each XCD then
-// holds one expert's four full tiles. False: no item for this work-group.
-__device__ __forceinline__ bool big_item(const GemmParams& p, int& tile, int& ct) {
+// at a cut). The narrow tiles come last in the table (tiles[1] = the number
+// before them), and each XCD takes its run of their items after its run of the
+// wide ones, so that what starts last is short. At M = 4096, E = 8, topk = 2
+// each XCD then holds one expert's four full tiles. False: no item for this
+// work-group.
+__device__ __forceinline__ bool gemm_item(const GemmParams& p, int& tile, int& ct, bool& narrow) {
   const int nt = p.tiles[0], nb = p.tiles[1];
   const int x = int(blockIdx.x) % kXcds;
   int s = int(blockIdx.x) / kXcds;
-  const int ib = nb * p.col_tiles, is = (nt - nb) * p.col_tiles;
+  const int ib = nb * p.col_tiles, is = (nt - nb) * p.narrow_cols;
   const int b0 = x * ib / kXcds, bn = (x + 1) * ib / kXcds - b0;
-  int item;
-  if (s < bn) {
-    item = b0 + s;
-  } else {
-    s -= bn;
-    const int s0 = x * is / kXcds;
-    if (s >= (x + 1) * is / kXcds - s0) return false;
-    item = ib + s0 + s;
+  narrow = s >= bn;
+  if (!narrow) {
+    s += b0;
+    tile = s / p.col_tiles;
+    ct = s % p.col_tiles;
+    return true;
   }
-  tile = item / p.col_tiles;
-  ct = item % p.col_tiles;
-  return true;
+  const int s0 = x * is / kXcds;
+  s += s0 - bn;
+  tile = nb + s / p.narrow_cols;
+  ct = s % p.narrow_cols;
+  return s < (x + 1) * is / kXcds;
 }
 
-// The K loop and epilogue of one wave's share of a big tile; NRB = its 32-pair
+// The K loop and epilogue of one wave's share of a tile; NRB = its 32-pair
 // row blocks holding pairs (0: DMAs and barriers only).
-template <bool kGated, int NRB>
-__device__ __forceinline__ void big_tile(const GemmParams& p, uint8_t* s_buf,
-                                         const uint8_t* abase, const uint8_t* wbase,
-                                         const uint32_t (&a_off)[4], const uint32_t (&b_off)[4],
-                                         uint32_t lds0, int na, int start, int rows, int ct) {
+template <bool kGated, TileForm kForm, int NRB>
+__device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* s_buf, int e, int start,
+                                         int rows, int ct) {
+  using L = TileLds<kForm>;
+  constexpr int kWq = L::kWq, kPh = L::kPh;
+  constexpr int kCols = L::kCols;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ph = wave >> 2;  // parity of the wave's row blocks
-  const int wq = wave & 3;   // weight quarter
+  const int ph = wave / kWq;  // the wave's row blocks: kPh * i + ph
+  const int wq = wave % kWq;  // weight part
   const int l32 = lane & 31;
   const int hi = lane >> 5;
   const int nst = p.kin / kBK;
   constexpr int kRB = NRB > 0 ? NRB : 1;
-  // DMAs of a stage: A groups 0..3 into A buffer `ab`, B groups 0..3 into B buffer `bb`
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)s_buf)));
+  const uint8_t* abase = reinterpret_cast<const uint8_t*>(p.a);
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.w + int64_t(e) * p.w_estride);
+
+  // Per-lane DMA sources: instruction g of this wave moves LDS rows
+  // 8 * (wave + 8 * g) + lane / 8, lane & 7 being the chunk position there.
+  const int sub = lane >> 3;
+  const int pos = lane & 7;
+  uint32_t a_off[L::kAGroups], b_off[L::kBGroups];
+  int64_t arow[L::kAGroups];
+#pragma unroll
+  for (int g = 0; g < L::kAGroups; ++g) {
+    const int r = 8 * (wave + 8 * g) + sub;
+    const int at = start + (r < rows ? r : 0);
+    arow[g] = kGated ? int64_t(p.sorted[at]) : int64_t(at);
+  }
+#pragma unroll
+  for (int g = 0; g < L::kAGroups; ++g) {
+    const int r = 8 * (wave + 8 * g) + sub;
+    if (kGated) arow[g] = uint32_t(arow[g]) / uint32_t(p.topk);
+    // the chunk whose swizzled position is `pos`
+    a_off[g] = uint32_t(arow[g] * p.a_stride * 2 + swz(r, pos) * 16);
+  }
+#pragma unroll
+  for (int g = 0; g < L::kBGroups; ++g) {
+    const int r = 8 * (wave + 8 * g) + sub;
+    // weight row of LDS row r: weight part r >> 6, column block (r >> 5) & 1
+    int wrow;
+    if (kGated)  // gate rows j, up rows N + j, j = ct * kCols / 2 + 32 * (r >> 6) + (r & 31)
+      wrow = (((r >> 5) & 1) ? p.nout : 0) + ct * (kCols / 2) + 32 * (r >> 6) + (r & 31);
+    else         // features f = ct * kCols + r
+      wrow = ct * kCols + r;
+    b_off[g] = uint32_t(int64_t(wrow) * p.kin * 2 + swz(r, pos) * 16);
+  }
+  // A instructions of this wave that hold a pair
+  const int na = max(0, min(L::kAGroups, (rows - 8 * wave + 63) / 64));
+  // DMAs of a stage: A group g into A buffer `ab`, B group g into B buffer `bb`
   auto dma_a = [&](int st, int ab, int g) {
     if (g < na)
       lds_dma(abase + int64_t(st) * kRowBytes, a_off[g],
-              lds0 + uint32_t(ab * kBigPart + (wave + 8 * g) * 1024));
+              lds0 + uint32_t(ab * L::kA + (wave + 8 * g) * 1024));
   };
   auto dma_b = [&](int st, int bb, int g) {
     lds_dma(wbase + int64_t(st) * kRowBytes, b_off[g],
-            lds0 + uint32_t((kBigABufs + bb) * kBigPart + (wave + 8 * g) * 1024));
+            lds0 + uint32_t(L::kABufs * L::kA + bb * L::kB + (wave + 8 * g) * 1024));
   };
 
   // the pairs of this lane's accumulator columns and their weights
@@ -858,7 +749,8 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, uint8_t* s_buf,
   float wt[kRB];
   if constexpr (!kGated && NRB > 0) {
 #pragma unroll
-    for (int rb = 0; rb < NRB; ++rb) pair[rb] = p.sorted[start + min(64 * rb + 32 * ph + l32, rows - 1)];
+    for (int rb = 0; rb < NRB; ++rb) 
+      pair[rb] = p.sorted[start + min(32 * (kPh * rb + ph) + l32, rows - 1)];
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb) wt[rb] = p.wts[pair[rb]];
   }
@@ -881,7 +773,8 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, uint8_t* s_buf,
       fr.b[f] = *reinterpret_cast<const bf16x8*>(sb + (64 * wq + 32 * f + l32) * kRowBytes + pos);
     else if (f - 2 < NRB)
       fr.a[f - 2] =
-          *reinterpret_cast<const bf16x8*>(sa + (32 * ph + 64 * (f - 2) + l32) * kRowBytes + pos);
+          *reinterpret_cast<const bf16x8*>(
+          sa + (32 * (kPh * (f - 2) + ph) + l32) * kRowBytes + pos);
   };
   // The MFMAs of step (fr), with the reads of the next step (sa, sb, kk) into
   // `nx` between them unless kk < 0; `after(i)` runs after MFMA pair i.
@@ -907,68 +800,83 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, uint8_t* s_buf,
 
   // nst >= 2: validate() requires K % 256 == 0 and N % 128 == 0
 #pragma unroll
-  for (int g = 0; g < 4; ++g) dma_a(0, 0, g);
+  for (int i = 0; i < L::kBBufs; ++i) {
+    if (i > 1 && i >= nst) break;
+    if (i < L::kABufs) {
 #pragma unroll
-  for (int g = 0; g < 4; ++g) dma_b(0, 0, g);
+      for (int g = 0; g < L::kAGroups; ++g) dma_a(i, i, g);
+    }
 #pragma unroll
-  for (int g = 0; g < 4; ++g) dma_a(1, 1, g);
-#pragma unroll
-  for (int g = 0; g < 4; ++g) dma_b(1, 1, g);
-  if (nst > 2) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) dma_b(2, 2, g);
+    for (int g = 0; g < L::kBGroups; ++g) dma_b(i, i, g);
   }
-  wait_vmcnt(na + (nst > 2 ? 8 : 4));
+  // DMAs of this wave issued after those of stage s when `ahead` stages of B
+  // follow it (fewer at the end): what may still fly once stage s has landed
+  auto later = [&](int s, int ahead) {
+    const int n = max(0, min(ahead, nst - 1 - s));
+    return n * (L::kABufs == L::kBBufs ? na + L::kBGroups : L::kBGroups);
+  };
+  // (the wide tile's counts, in the loop: 4 or 0)
+  auto wait_stage = [&](int s) {
+    if constexpr (kForm != kWide) {
+      wait_vmcnt(later(s, L::kBBufs - 2));
+    } else {
+      if (s + 1 < nst)
+        wait_vmcnt(L::kBGroups);
+      else
+        wait_vmcnt(0);
+    }
+  };
+  // (wide: A of stage 1 too)
+  wait_vmcnt(later(0, L::kBBufs - 1) + (L::kABufs < L::kBBufs ? na : 0));
   lds_barrier();
-  const uint8_t* const sb0 = s_buf + kBigABufs * kBigPart;
+  const uint8_t* const sb0 = s_buf + L::kABufs * L::kA;
   Frags f0, f1;
 #pragma unroll
   for (int f = 0; f < NRB + 2; ++f) read1(s_buf, sb0, 0, f, f0);
-  int bb = 0;  // st % 3
+  int ab = 0, bb = 0;  // the buffers of stage st
   for (int st = 0; st < nst; ++st) {
-    const uint8_t* sa = s_buf + (st & 1) * kBigPart;
-    const uint8_t* sb = sb0 + bb * kBigPart;
-    const int nb = bb == kBigBBufs - 1 ? 0 : bb + 1;
+    const uint8_t* sa = s_buf + ab * L::kA;
+    const uint8_t* sb = sb0 + bb * L::kB;
+    const int na1 = ab == L::kABufs - 1 ? 0 : ab + 1, nb1 = bb == L::kBBufs - 1 ? 0 : bb + 1;
     step(f0, sa, sb, 1, f1, nothing);
     step(f1, sa, sb, 2, f0, nothing);
     step(f0, sa, sb, 3, f1, nothing);
-    // stage st + 1 has landed (only the weights of stage st + 2 still fly), then
-    // it has for every wave, and every wave has read stage st (the last pass
-    // reads a stale stage ahead, unused)
-    if (st + 2 < nst)
-      wait_vmcnt(4);
-    else
-      wait_vmcnt(0);
+    // stage st + 1 has landed, then it has for every wave, and every wave has
+    // read stage st (the last pass reads a stale stage ahead, unused)
+    wait_stage(st + 1);
     lds_barrier();
-    // the DMAs into stage st's buffers: A of stage st + 2, B of stage st + 3
-    const bool ma = st + 2 < nst, mb = st + 3 < nst;
+    // the DMAs into stage st's buffers
+    const bool ma = st + L::kABufs < nst, mb = st + L::kBBufs < nst;
     auto dmas = [&](int rb) {
+      constexpr int kN = L::kAGroups + L::kBGroups;
 #pragma unroll
-      for (int d = rb * 8 / kRB; d < (rb + 1) * 8 / kRB; ++d) {
-        if (d < 4) {
-          if (ma) dma_a(st + 2, st & 1, d);
+      for (int d = rb * kN / kRB; d < (rb + 1) * kN / kRB; ++d) {
+        if (d < L::kAGroups) {
+          if (ma) dma_a(st + L::kABufs, ab, d);
         } else {
-          if (mb) dma_b(st + 3, bb, d - 4);
+          if (mb) dma_b(st + L::kBBufs, bb, d - L::kAGroups);
         }
       }
     };
     if constexpr (NRB == 0) dmas(0);
-    step(f1, s_buf + ((st + 1) & 1) * kBigPart, sb0 + nb * kBigPart, 0, f0, dmas);
-    bb = nb;
+    step(f1, s_buf + na1 * L::kA, sb0 + nb1 * L::kB, 0, f0, dmas);
+    ab = na1;
+    bb = nb1;
   }
 
-  // epilogue: the lane holds, for pair row 64 * rb + 32 * ph + l32, weight rows
+  // epilogue: the lane holds, for pair row 32 * (kPh * rb + ph) + l32, weight
+  // rows
   // 8 * a + 4 * hi + i of each column block in register 4 * a + i. The outputs
   // go through this wave's own LDS lines, so that global stores write 64
   // (gated) or 128 contiguous bytes of a row by 16 bytes per lane: 2 us instead
   // of 5 for 2-byte stores straight from the accumulators.
   lds_barrier();  // every wave's reads are done
   if constexpr (NRB > 0) {
-    constexpr int kPitch = kGated ? kBigPitchGated : kBigPitchDown;
+    constexpr int kPitch = kGated ? kPitchGated : kPitchDown;
     constexpr int kOuts = kGated ? 32 : 64;        // outputs per pair row and wave
     constexpr int kLanes = kOuts / 8;              // lanes per row of a 16-byte store
-    uint8_t* const sw = s_buf + wave * (128 * kBigPitchDown);
-    int* const sp = reinterpret_cast<int*>(s_buf + kBigPairs) + 128 * wave;
+    uint8_t* const sw = s_buf + wave * (128 * kPitchDown);
+    int* const sp = reinterpret_cast<int*>(s_buf + kPairsOff) + 128 * wave;
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb) {
       uint8_t* line = sw + (32 * rb + l32) * kPitch + 8 * hi;
@@ -1000,79 +908,59 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, uint8_t* s_buf,
 #pragma unroll
     for (int i = 0; i < 32 * NRB / (64 / kLanes); ++i) {
       const int lr = i * (64 / kLanes) + lane / kLanes;     // row within the wave's
-      const int r = 64 * (lr >> 5) + 32 * ph + (lr & 31);   // row of the tile
+      const int r = 32 * (kPh * (lr >> 5) + ph) + (lr & 31);  // row of the tile
       if (r >= rows) continue;
       const bf16x8 v = *reinterpret_cast<const bf16x8*>(sw + lr * kPitch + 16 * c);
-      __bf16* dst;
-      if constexpr (kGated)
-        dst = p.out + int64_t(start + r) * p.out_stride + ct * (kLargeCols / 2) + 32 * wq;
-      else
-        dst = p.out + int64_t(sp[lr]) * p.out_stride + ct * kLargeCols + 64 * wq;
-      *reinterpret_cast<bf16x8*>(dst + 8 * c) = v;
+      if constexpr (kGated) {
+        __bf16* dst = p.out + int64_t(start + r) * p.out_stride + ct * (kCols / 2) + 32 * wq;
+        *reinterpret_cast<bf16x8*>(dst + 8 * c) = v;
+      } else {
+        const int f = ct * kCols + 64 * wq + 8 * c;
+        if (p.fsum != nullptr) {
+          __bf16* dst = p.fsum + int64_t(uint32_t(sp[lr]) / uint32_t(p.topk)) * p.fsum_stride + f;
+#pragma unroll
+          for (int j = 0; j < 8; j += 2) add_bf16x2(dst + j, v[j], v[j + 1]);
+        } else {
+          *reinterpret_cast<bf16x8*>(p.out + int64_t(sp[lr]) * p.out_stride + f) = v;
+        }
+      }
     }
   }
 }
 
 template <bool kGated>
-__global__ void __launch_bounds__(512, 1) fm_gemm_big_kernel(const GemmParams p) {
-  __shared__ __attribute__((aligned(1024))) uint8_t s_buf[kBigLds];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
+__global__ void __launch_bounds__(512, 1) fm_gemm_kernel(const GemmParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t s_buf[kGemmLds];
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   int tile, ct;
-  if (!big_item(p, tile, ct)) return;
+  bool narrow;
+  if (!gemm_item(p, tile, ct, narrow)) return;
   const int32_t* tl = p.tiles + 4 + 4 * tile;
   const int e = __builtin_amdgcn_readfirstlane(tl[0]);
   const int start = __builtin_amdgcn_readfirstlane(tl[1]);
   const int rows = __builtin_amdgcn_readfirstlane(tl[2]);
-
-  // Per-lane DMA sources: instruction g of this wave moves LDS rows
-  // 8 * (wave + 8 * g) + lane / 8, lane & 7 being the chunk position there.
-  const int sub = lane >> 3;
-  const int pos = lane & 7;
-  uint32_t a_off[4], b_off[4];
-  int64_t arow[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int r = 8 * (wave + 8 * g) + sub;
-    const int at = start + (r < rows ? r : 0);
-    arow[g] = kGated ? int64_t(p.sorted[at]) : int64_t(at);
+  if (narrow) {  // wave w: row block w
+    if (rows <= 128) {
+      if (32 * wave < rows)
+        gemm_tile<kGated, kNarrow128, 1>(p, s_buf, e, start, rows, ct);
+      else
+        gemm_tile<kGated, kNarrow128, 0>(p, s_buf, e, start, rows, ct);
+    } else {
+      if (32 * wave < rows)
+        gemm_tile<kGated, kNarrow256, 1>(p, s_buf, e, start, rows, ct);
+      else
+        gemm_tile<kGated, kNarrow256, 0>(p, s_buf, e, start, rows, ct);
+    }
+    return;
   }
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int r = 8 * (wave + 8 * g) + sub;
-    const int c = swz(r, pos);  // the chunk whose swizzled position is `pos`
-    if (kGated) arow[g] = uint32_t(arow[g]) / uint32_t(p.topk);
-    a_off[g] = uint32_t(arow[g] * p.a_stride * 2 + c * 16);
-    // weight row of LDS row r: weight quarter r >> 6, column block (r >> 5) & 1
-    int wrow;
-    if (kGated)  // gate rows j, up rows N + j, j = ct * 128 + 32 * (r >> 6) + (r & 31)
-      wrow = (((r >> 5) & 1) ? p.nout : 0) + ct * (kLargeCols / 2) + 32 * (r >> 6) + (r & 31);
-    else         // features f = ct * 256 + r
-      wrow = ct * kLargeCols + r;
-    b_off[g] = uint32_t(int64_t(wrow) * p.kin * 2 + c * 16);
-  }
-  // A instructions of this wave that hold a pair
-  const int na = max(0, min(4, (rows - 8 * wave + 63) / 64));
-  const uint8_t* abase = reinterpret_cast<const uint8_t*>(p.a);
-  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.w + int64_t(e) * p.w_estride);
-  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
-      uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)s_buf)));
-
   // 32-pair row blocks 2 i + (wave >> 2) that hold pairs
-  const int nrb = max(0, min(4, (rows - 32 * (wave >> 2) + 63) / 64));
-#define FM_BIG(n) \
-  big_tile<kGated, n>(p, s_buf, abase, wbase, a_off, b_off, lds0, na, start, rows, ct)
-  switch (nrb) {
-    case 0: FM_BIG(0); break;
-    case 1: FM_BIG(1); break;
-    case 2: FM_BIG(2); break;
-    case 3: FM_BIG(3); break;
-    default: FM_BIG(4); break;
+  switch (max(0, min(4, (rows - 32 * (wave >> 2) + 63) / 64))) {
+    case 0: gemm_tile<kGated, kWide, 0>(p, s_buf, e, start, rows, ct); break;
+    case 1: gemm_tile<kGated, kWide, 1>(p, s_buf, e, start, rows, ct); break;
+    case 2: gemm_tile<kGated, kWide, 2>(p, s_buf, e, start, rows, ct); break;
+    case 3: gemm_tile<kGated, kWide, 3>(p, s_buf, e, start, rows, ct); break;
+    default: gemm_tile<kGated, kWide, 4>(p, s_buf, e, start, rows, ct); break;
   }
-#undef FM_BIG
 }
 
 // ---- skinny tiles (few pairs per expert) ------------------------------------------
@@ -1464,11 +1352,12 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   rp.E = int(a->E);
   rp.topk = int(a->topk);
   rp.renormalize = a->renormalize ? 1 : 0;
-  // With at most two experts per token, the down GEMM of streamed tiles adds
-  // into the output itself and the routing launch clears it: no final-sum
-  // launch.
-  const bool streamed = !pl.large && a->N % kStK == 0;  // (K % 256 == 0 always holds)
-  const bool fsum = streamed && a->topk <= 2 && (a->flags & FM_FLAG_ORDERED_SUM) == 0;
+  // With at most two experts per token, the down GEMM of streamed tiles, or of
+  // up to 24 pairs per expert, adds into the output itself and the routing
+  // launch clears it: no final-sum launch.
+  const bool streamed = !pl.gemm && a->N % kStK == 0;  // (K % 256 == 0 always holds)
+  const bool fsum = a->topk <= 2 && (a->flags & FM_FLAG_ORDERED_SUM) == 0 &&
+                    (streamed || (pl.gemm && a->N % kStK == 0 && pl.P <= 24 * a->E));
   if (fsum) {
     rp.zero_out = static_cast<__bf16*>(a->out);
     rp.s_out = a->s_out;
@@ -1482,8 +1371,7 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   pp.P = pl.P;
   pp.E = int(a->E);
   pp.tile_rows = pl.tile_rows;
-  // big tiles with at most two gate-up items per CU: what starts last is short
-  pp.split_small = pl.big && pl.max_tiles * (a->N / (kLargeCols / 2)) <= 512;
+  pp.narrow_rows = pl.narrow_rows;
   if (a->M <= kFusedRouteTokens) {  // one launch, reported as the plan's
     void* ka[] = {&rp, &pp};
     if (!run(FM_KERNEL_PLAN, fn(fm_route_plan_kernel), dim3(1), dim3(1024), ka)) return FM_EHIP;
@@ -1517,9 +1405,11 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   g2.out_stride = a->K;
   g2.kin = int(a->N);
   g2.nout = int(a->K);
-  if (pl.large) {
-    g1.col_tiles = int(a->N / (kLargeCols / 2));
-    g2.col_tiles = int(a->K / kLargeCols);
+  if (pl.gemm) {
+    g1.col_tiles = int(a->N / (kTileCols / 2));
+    g2.col_tiles = int(a->K / kTileCols);
+    g1.narrow_cols = int(a->N / (kNarrowCols / 2));
+    g2.narrow_cols = int(a->K / kNarrowCols);
   } else {
     g1.col_tiles = int(a->N / 16);
     g2.col_tiles = int(a->K / 32);
@@ -1531,11 +1421,6 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
     g2.fsum_stride = a->s_out;
   }
   g1.ct_per_wg = g2.ct_per_wg = 1;
-  // (MI355X: 256 CUs, one large work-group each)
-  const double pairs_per_expert = double(pl.P) / double(a->E);
-  for (GemmParams* g : {&g1, &g2})
-    g->xcd_grid = pl.large && pairs_per_expert < 2.0 * pl.tile_rows &&
-                  pl.max_tiles * g->col_tiles > 256;
   if (streamed) {
     // a streaming work-group runs several column tiles in one pipeline, so its
     // start (tile table -> pair list -> first DMA) is paid once per
@@ -1547,11 +1432,14 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
     }
   }
   auto grid_of = [&](const GemmParams& g) {
-    if (pl.big)  // big_item: each XCD has at most 1 / 8 of the items of each size, rounded up
-      return unsigned(kXcds * (pl.max_tiles * g.col_tiles / kXcds + 2));
-    if (pl.large)  // xcd_item: each XCD has up to ceil(tiles / 4) x ceil(col_tiles / 2) items
-      return unsigned(kXcds * ((pl.max_tiles + kXcdTileGroups - 1) / kXcdTileGroups) *
-                      ((g.col_tiles + kXcdColGroups - 1) / kXcdColGroups));
+    if (pl.gemm) {  // gemm_item: an XCD has at most 1 / 8 of the items of each kind, rounded up
+      const bool all = pl.tile_rows <= pl.narrow_rows;  // every tile is narrow
+      const int64_t narrow = all ? pl.max_tiles : pl.narrow_rows > 0 ? pl.nonempty : 0;
+      // (a wide tile holds more than narrow_rows pairs)
+      const int64_t wide =
+          all ? 0 : std::min<int64_t>(pl.max_tiles, pl.P / (pl.narrow_rows + 1));
+      return unsigned(kXcds * ((wide * g.col_tiles + narrow * g.narrow_cols) / kXcds + 2));
+    }
     return unsigned(pl.max_tiles * ((g.col_tiles + g.ct_per_wg - 1) / g.ct_per_wg));
   };
   const unsigned grid1 = grid_of(g1);
@@ -1559,14 +1447,13 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   // the GEMM kernel of this plan, gated (gate-up) or not (down)
   auto gemm = [&](auto gated) -> const void* {
     constexpr bool G = decltype(gated)::value;
-    if (pl.big) return fn(fm_gemm_big_kernel<G>);
-    if (pl.large) return fn(fm_gemm_kernel<G>);
+    if (pl.gemm) return fn(fm_gemm_kernel<G>);
     if (streamed)
       return pl.pb == 1 ? fn(fm_stream_kernel<G, 1>)
                         : pl.pb == 2 ? fn(fm_stream_kernel<G, 2>) : fn(fm_stream_kernel<G, 4>);
     return pl.pb == 1 ? fn(fm_skinny_kernel<G, 1>) : fn(fm_skinny_kernel<G, 2>);
   };
-  const dim3 gemm_block(pl.big ? 512 : 256);
+  const dim3 gemm_block(pl.gemm ? 512 : 256);
   void* k1[] = {&g1};
   if (!run(FM_KERNEL_GATEUP, gemm(std::true_type{}), dim3(grid1), gemm_block, k1)) return FM_EHIP;
   void* k2[] = {&g2};

@@ -158,21 +158,33 @@ def test_big_tiles_equal_large_tiles(gpu_sa, shape):
 
 
 @pytest.mark.parametrize("counts,K,N", [
-    ((1, 32, 33, 64), 256, 128), ((65, 128, 129, 0, 255), 256, 128),
-    ((256, 257, 384, 385, 512, 640), 512, 128), ((300,) * 20 + (100,) * 44, 256, 2048)])
-def test_big_tiles_at_their_edges(gpu_sa, counts, K, N):
-    """256-pair tiles of every filling (row blocks of one or both wave halves,
-    DMA groups partly past the last pair), with the small ones listed last
-    (up to 512 work items) and in the experts' order (more), against the
-    128-pair tiles: the same MFMA sequence per output element, so the same
-    bits."""
+    ((1, 32, 33, 64), 256, 128), ((65, 128, 129, 0, 255, 256), 256, 128),
+    ((256, 257, 384, 385, 512, 640), 512, 128), ((300,) * 20 + (100,) * 44, 256, 2048),
+    ((17, 200, 256, 31) * 8, 512, 640)])
+def test_gemm_tiles_at_their_edges(gpu_sa, counts, K, N):
+    """Wide and narrow tiles of every filling (row blocks of one or both wave
+    halves, DMA groups partly past the last pair, short last tiles narrow or
+    wide, every tile narrow), as chosen and with 256- and 128-pair tiles: the
+    same MFMA sequence per output element, so the same bits; and the oracle."""
     E, M = len(counts), sum(counts)
     hidden, w1, w2, _ = make_inputs(M, K, N, E, seed=11)
     ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
     ids = ids[torch.randperm(M, generator=torch.Generator().manual_seed(12))].to(DEV)
     score = torch.nn.functional.one_hot(ids, E).to(torch.bfloat16) * 4
-    big = op(hidden, w1, w2, score, 1, flags=4)
-    assert torch.equal(big, op(hidden, w1, w2, score, 1, flags=1))
+    out = op(hidden, w1, w2, score, 1)
+    assert torch.equal(out, op(hidden, w1, w2, score, 1, flags=4))
+    assert torch.equal(out, op(hidden, w1, w2, score, 1, flags=1))
+    check(out, fused_moe_ref(*cpu(hidden, w1, w2, score), 1), f"{counts[:6]}")
+
+
+@pytest.mark.parametrize("M", [16, 64])
+def test_streamed_final_sum_forms(gpu_sa, M):
+    """Streamed tiles where fm_gemm_kernel is the default: the atomic and the
+    ordered final sum give the same bits."""
+    hidden, w1, w2, score = make_inputs(M, 2048, 1024, 8, seed=13)
+    out = op(hidden, w1, w2, score, 2, flags=2)
+    assert torch.equal(out, op(hidden, w1, w2, score, 2, flags=2 | 8))
+    check(out, fused_moe_ref(*cpu(hidden, w1, w2, score), 2), f"streamed M={M}")
 
 
 @pytest.mark.parametrize("shape", [(37, 256, 128, 4, 4), (5, 256, 128, 1, 1), (1, 256, 128, 256, 32),
