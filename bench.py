@@ -579,7 +579,7 @@ MOE_WORKLOADS = [  # track-03/workloads.py:3-12: label, M, K, N, E, topk
 ]
 MOE_KERNEL_NAMES = {"route": "fm_route_kernel", "plan": "fm_plan_kernel",
                     "reduce": "fm_reduce_kernel"}
-MOE_FUSED_ROUTE_TOKENS = 16  # kFusedRouteTokens in csrc/fused_moe_gfx950.hip
+MOE_FUSED_ROUTE_TOKENS = 16  # kFusedTokens in csrc/fused_moe_gfx950.hip
 
 
 def moe_gemm_kernel(M, N, E, topk, gated):

@@ -14,9 +14,11 @@
 // -------------------
 // fm_route_kernel   one wave per token: softmax over E, top-k by repeated
 //   wave-wide argmax on (weight, lower index), ids and bf16 weights written
-//   in ascending expert order (the order of the final sum).
-// fm_plan_kernel    one work-group: pairs (t, slot) counted per expert and
-//   listed by expert, tiles of up to `tile_rows` pairs of one expert.
+//   in ascending expert order (the order of the final sum), and each
+//   work-group's pairs counted per expert.
+// fm_plan_kernel    as many work-groups: pairs (t, slot) listed by expert,
+//   tiles of up to `tile_rows` pairs of one expert. Up to 16 tokens both are
+//   one work-group's work (fm_route_plan_kernel).
 // fm_gemm_kernel<gated>   (prefill, and decode over few experts) a tile of up
 //   to 256 pairs x 256 weight rows (wide) or 64 (narrow) per work-group, K in
 //   64-wide stages through LDS rings filled by LDS-DMA (1 KiB per wave
@@ -56,6 +58,7 @@ typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
 
 constexpr int kMaxExperts = 256;
 constexpr int kMaxTopk = 32;
+constexpr int kFusedTokens = 16;  // routing and plan in one launch up to this many tokens
 
 // ---------------------------------------------------------------------------
 // workspace plan (host)
@@ -76,7 +79,8 @@ struct Plan {
   int narrow_rows;      // gemm: tiles of at most this many pairs run as narrow ones
   int pb;               // not gemm: 16-pair blocks per tile (1, 2 or 4)
   int64_t max_tiles;    // upper bound on sum_e ceil(count_e / tile_rows)
-  size_t ids_off, wts_off, eoff_off, sorted_off, tiles_off, inter_off, y_off, bytes;
+  int tokens_per_wg, route_wgs;  // fm_route_kernel: at most 256 work-groups (0: fused)
+  size_t ids_off, wts_off, hist_off, sorted_off, tiles_off, inter_off, y_off, bytes;
 };
 
 inline size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -142,6 +146,8 @@ Plan make_plan(const fm_args* a) {
   p.nonempty = a->E < p.P ? a->E : p.P;
   choose_tiles(a, p);
   p.max_tiles = p.P / p.tile_rows + p.nonempty;
+  p.tokens_per_wg = int((a->M + 4095) / 4096) * 16;
+  p.route_wgs = a->M <= kFusedTokens ? 0 : int((a->M + p.tokens_per_wg - 1) / p.tokens_per_wg);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -150,7 +156,7 @@ Plan make_plan(const fm_args* a) {
   };
   p.ids_off = take(size_t(p.P) * 4);
   p.wts_off = take(size_t(p.P) * 4);
-  p.eoff_off = take(size_t(a->E + 1) * 4);
+  p.hist_off = take(size_t(p.route_wgs) * size_t(a->E) * 4);
   p.sorted_off = take(size_t(p.P) * 4);
   p.tiles_off = take(16 + size_t(p.max_tiles) * 16);  // count, then int4 per tile
   p.inter_off = take(size_t(p.P) * size_t(a->N) * 2);
@@ -209,13 +215,20 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const unsigned long long y = __shfl_xor(x, o);
-    x = y > x ? y : x;
-  }
-  return x;
+// Largest of the 64 lanes' values, in every lane: DPP moves within the rows of
+// 16 lanes, then across them (six dependent VALU steps; a 64-bit shuffle
+// butterfly took two LDS round trips per step).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+#define FM_DPP_MAX(ctrl, rows) \
+  x = max(x, uint32_t(__builtin_amdgcn_update_dpp(int(x), int(x), ctrl, rows, 0xf, false)))
+  FM_DPP_MAX(0x111, 0xf);  // row_shr:1, 2, 4, 8: lane 15 of a row holds the row's maximum
+  FM_DPP_MAX(0x112, 0xf);
+  FM_DPP_MAX(0x114, 0xf);
+  FM_DPP_MAX(0x118, 0xf);
+  FM_DPP_MAX(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  FM_DPP_MAX(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef FM_DPP_MAX
+  return uint32_t(__builtin_amdgcn_readlane(int(x), 63));
 }
 
 // LDS-DMA of 16 bytes per lane from SGPR base + 32-bit lane offset into
@@ -279,9 +292,11 @@ __device__ __forceinline__ void wait_vmcnt(int n) {  // n uniform, 0..24
 struct RouteParams {
   const __bf16* score;
   int64_t s_score;
-  int32_t* ids;     // [M, topk] ascending expert ids
+  int32_t* ids;     // [M, topk] ascending expert ids; bits 8..31: see fm_route_kernel
   float* wts;       // [M, topk] bf16-rounded weights (as fp32)
+  int32_t* hist;    // [work-groups, E] pairs per expert of a work-group's tokens
   int64_t M;
+  int tokens_per_wg;
   int E, topk, renormalize;
   // when the down GEMM adds into the output itself: the rows to clear
   __bf16* zero_out;
@@ -298,9 +313,11 @@ __device__ __forceinline__ void clear_out_row(const RouteParams& p, int64_t t, i
   for (int k = 8 * lane; k < p.K; k += 8 * 64) *reinterpret_cast<bf16x8*>(row + k) = z;
 }
 
-// Routing of token t by one wave; lane l holds experts l, l + 64, l + 128,
-// l + 192. `raw` are the token's scores as loaded (bf16 widened; -inf past E).
-constexpr int kPer = kMaxExperts / 64;
+// Routing of token t by one wave; lane l holds experts l + 64 i, i < kPer
+// (kPer = 1 for E <= 64, else 4). `raw` are the token's scores as loaded (bf16
+// widened; -inf past E). `id(slot, e)` takes the selected experts in ascending
+// order of e, one call by the lane that holds e.
+template <int kPer>
 __device__ __forceinline__ void load_scores(const RouteParams& p, int64_t t, int lane,
                                             float (&raw)[kPer]) {
   const __bf16* srow = p.score + t * p.s_score;
@@ -311,8 +328,9 @@ __device__ __forceinline__ void load_scores(const RouteParams& p, int64_t t, int
   }
 }
 
+template <int kPer, typename Id>
 __device__ __forceinline__ void route_token(const RouteParams& p, int64_t t, int lane,
-                                            const float (&raw)[kPer]) {
+                                            const float (&raw)[kPer], Id id) {
   float v[kPer];
   float mx = -INFINITY;
 #pragma unroll
@@ -330,27 +348,28 @@ __device__ __forceinline__ void route_token(const RouteParams& p, int64_t t, int
   sum = wave_sum(sum);
 #pragma unroll
   for (int i = 0; i < kPer; ++i) v[i] = v[i] / sum;  // softmax weight (>= 0)
-  // top-k: repeated argmax over (weight, lower index); a weight's bits order
-  // like its value (weights are >= 0), the index goes in complemented
+  // top-k: repeated argmax over (weight, lower index). A weight's bits order
+  // like its value (weights are >= 0); among equal ones the lowest lane of the
+  // lowest i is the lowest expert.
   bool sel[kPer] = {};
   float tot = 0.f;  // sum of the selected weights, in selection order
   for (int r = 0; r < p.topk; ++r) {
-    unsigned long long key = 0ull;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int e = lane + 64 * i;
-      if (e < p.E && !sel[i]) {
-        const unsigned long long k = (static_cast<unsigned long long>(__float_as_uint(v[i])) << 32) |
-                                     (0xFFFFFFFFu - unsigned(e));
-        key = k > key ? k : key;
-      }
-    }
-    key = wave_max_u64(key);
-    const int win = int(0xFFFFFFFFu - unsigned(key & 0xFFFFFFFFull));
-    tot += __uint_as_float(unsigned(key >> 32));
+    uint32_t key = 0u;
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
-      if (lane + 64 * i == win) sel[i] = true;
+      if (!sel[i] && lane + 64 * i < p.E) key = max(key, __float_as_uint(v[i]));
+    key = wave_max_u32(key);
+    tot += __uint_as_float(key);
+    bool found = false;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const unsigned long long m =
+          __ballot(!sel[i] && lane + 64 * i < p.E && __float_as_uint(v[i]) == key);
+      if (!found && m != 0ull) {
+        found = true;
+        if (lane == __builtin_ctzll(m)) sel[i] = true;
+      }
+    }
   }
   // ascending-expert slot of each selected expert: ballots in expert order
   int before = 0;
@@ -361,34 +380,50 @@ __device__ __forceinline__ void route_token(const RouteParams& p, int64_t t, int
     if (sel[i]) {
       const int slot = before + __popcll(m & below);
       const float w = p.renormalize ? v[i] / tot : v[i];
-      p.ids[t * p.topk + slot] = lane + 64 * i;
+      id(slot, lane + 64 * i);
       p.wts[t * p.topk + slot] = bf16r(w);
     }
     before += __popcll(m);
   }
 }
 
-// One wave per token.
-__global__ void __launch_bounds__(256) fm_route_kernel(const RouteParams p) {
+// One wave per token, 16 at a time per work-group. Besides its expert a pair
+// gets its rank among the work-group's pairs of that expert (bits 8..31 of the
+// id), and the work-group's counts go to `hist`: the plan then needs no
+// atomics over all pairs.
+constexpr int kRouteWaves = 16;
+template <int kPer>
+__global__ void __launch_bounds__(64 * kRouteWaves) fm_route_kernel(const RouteParams p) {
+  __shared__ int s_cnt[kMaxExperts];
   const int lane = threadIdx.x & 63;
-  const int64_t t = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (t >= p.M) return;
-  float raw[kPer];
-  load_scores(p, t, lane, raw);
-  route_token(p, t, lane, raw);
-  if (p.zero_out != nullptr) clear_out_row(p, t, lane);
+  const int64_t t0 = int64_t(blockIdx.x) * p.tokens_per_wg;
+  const int64_t t1 = t0 + p.tokens_per_wg < p.M ? t0 + p.tokens_per_wg : p.M;
+  for (int e = threadIdx.x; e < p.E; e += 64 * kRouteWaves) s_cnt[e] = 0;
+  __syncthreads();
+  for (int64_t t = t0 + (threadIdx.x >> 6); t < t1; t += kRouteWaves) {
+    float raw[kPer];
+    load_scores(p, t, lane, raw);
+    route_token(p, t, lane, raw, [&](int slot, int e) {
+      p.ids[t * p.topk + slot] = e | atomicAdd(&s_cnt[e], 1) << 8;
+    });
+    if (p.zero_out != nullptr) clear_out_row(p, t, lane);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < p.E; e += 64 * kRouteWaves)
+    p.hist[int64_t(blockIdx.x) * p.E + e] = s_cnt[e];
 }
 
 // ============================================================================
 // plan: pairs by expert, tiles
 // ============================================================================
 struct PlanParams {
-  const int32_t* ids;
-  int32_t* eoff;      // [E + 1] first sorted position of each expert
+  const int32_t* ids;   // fm_route_kernel's
+  const int32_t* hist;
   int32_t* sorted;    // [P] pair ids (t * topk + slot) grouped by expert
   int32_t* tiles;     // [0] = tile count, [1] = tiles before the narrow ones, then
                       // int4 (expert, start, rows, 0) per tile
   int64_t P;
+  int wgs, pairs_per_wg;  // of fm_route_kernel
   int E, tile_rows;
   int narrow_rows;    // tiles of at most this many pairs are listed last (narrow tiles)
 };
@@ -401,128 +436,169 @@ struct PlanSmem {
   int cur[kMaxExperts];
 };
 
-// The plan, by the 1024 threads of one work-group.
-__device__ __forceinline__ void plan_body(const PlanParams& p, PlanSmem& sm) {
-  int* s_cnt = sm.cnt;
-  int* s_off = sm.off;
-  int* s_toff = sm.toff;
-  int* s_soff = sm.soff;
-  // tiles of an expert with n pairs, and how many of them (the last one, or
-  // all) are narrow
-  // (tile_rows is a power of two)
-  const int log_rows = __builtin_ctz(p.tile_rows);
-  auto tiles_of = [&](int n) { return (n + p.tile_rows - 1) >> log_rows; };
-  auto narrow_of = [&](int n) {
-    const int nt = tiles_of(n);
-    return p.tile_rows <= p.narrow_rows ? nt
-                                        : n > 0 && n - (nt - 1) * p.tile_rows <= p.narrow_rows;
-  };
-  int* s_cur = sm.cur;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < kMaxExperts; e += 1024) {
-    s_cnt[e] = 0;
-    s_cur[e] = 0;
-  }
-  __syncthreads();
-  for (int64_t i = tid; i < p.P; i += 1024) atomicAdd(&s_cnt[p.ids[i]], 1);
-  __syncthreads();
-  if (tid < 64) {  // exclusive scans of counts and tile counts over <= 256 experts
-    int carry = 0, tcarry = 0, scarry = 0;
-    for (int c = 0; c < kMaxExperts / 64; ++c) {
-      const int e = 64 * c + tid;
-      const int v = e < p.E ? s_cnt[e] : 0;
-      const int sv = narrow_of(v);
-      const int tv = tiles_of(v) - sv;
-      int incl = v, tincl = tv, sincl = sv;
+// Tiles of an expert with n pairs (tile_rows is a power of two), and how many
+// of them (the last one, or all) are narrow.
+__device__ __forceinline__ int tiles_of(const PlanParams& p, int n) {
+  return (n + p.tile_rows - 1) >> __builtin_ctz(p.tile_rows);
+}
+__device__ __forceinline__ int narrow_of(const PlanParams& p, int n) {
+  const int nt = tiles_of(p, n);
+  return p.tile_rows <= p.narrow_rows ? nt
+                                      : n > 0 && n - (nt - 1) * p.tile_rows <= p.narrow_rows;
+}
+
+// Exclusive scans over the experts, by wave 0, from their counts: first sorted
+// position, first wide and first narrow tile.
+__device__ __forceinline__ void plan_scan(const PlanParams& p, PlanSmem& sm) {
+  const int lane = threadIdx.x;
+  int carry = 0, tcarry = 0, scarry = 0;
+  for (int e0 = 0; e0 < p.E; e0 += 64) {
+    const int e = e0 + lane;
+    const int v = e < p.E ? sm.cnt[e] : 0;
+    const int sv = narrow_of(p, v);
+    const int tv = tiles_of(p, v) - sv;
+    int incl = v, tincl = tv, sincl = sv;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int a = __shfl_up(incl, o);
+      const int b = __shfl_up(tincl, o);
+      if (lane >= o) {
+        incl += a;
+        tincl += b;
+      }
+    }
+    if (p.narrow_rows > 0) {
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
-        const int a = __shfl_up(incl, o);
-        const int b = __shfl_up(tincl, o);
-        if (tid >= o) {
-          incl += a;
-          tincl += b;
-        }
+        const int d = __shfl_up(sincl, o);
+        if (lane >= o) sincl += d;
       }
-      if (p.narrow_rows > 0) {
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int d = __shfl_up(sincl, o);
-          if (tid >= o) sincl += d;
-        }
-      }
-      if (e < p.E) {
-        s_off[e] = carry + incl - v;
-        s_toff[e] = tcarry + tincl - tv;
-        s_soff[e] = scarry + sincl - sv;
-      }
-      carry += __shfl(incl, 63);
-      tcarry += __shfl(tincl, 63);
-      scarry += __shfl(sincl, 63);
     }
-    if (tid == 0) {
-      s_off[p.E] = carry;
-      s_toff[p.E] = tcarry;
-      s_soff[p.E] = scarry;
+    if (e < p.E) {
+      sm.off[e] = carry + incl - v;
+      sm.toff[e] = tcarry + tincl - tv;
+      sm.soff[e] = scarry + sincl - sv;
     }
+    carry += __shfl(incl, 63);
+    tcarry += __shfl(tincl, 63);
+    scarry += __shfl(sincl, 63);
   }
-  __syncthreads();
-  for (int e = tid; e <= p.E; e += 1024) p.eoff[e] = s_off[e];
+  if (lane == 0) {
+    sm.toff[p.E] = tcarry;
+    sm.soff[p.E] = scarry;
+  }
+}
+
+// The tile table, by the 1024 threads of one work-group, after the scan.
+__device__ __forceinline__ void plan_tiles(const PlanParams& p, const PlanSmem& sm) {
+  const int tid = threadIdx.x;
   if (tid == 0) {
-    p.tiles[0] = s_toff[p.E] + s_soff[p.E];
-    p.tiles[1] = s_toff[p.E];
+    p.tiles[0] = sm.toff[p.E] + sm.soff[p.E];
+    p.tiles[1] = sm.toff[p.E];
   }
-  for (int64_t i = tid; i < p.P; i += 1024) {
-    const int e = p.ids[i];
-    p.sorted[s_off[e] + atomicAdd(&s_cur[e], 1)] = int32_t(i);
-  }
-  for (int e = tid; e < p.E; e += 1024) {
-    const int n = s_cnt[e];
-    for (int k = 0; k * p.tile_rows < n; ++k) {
-      const int wide = tiles_of(n) - narrow_of(n);
-      const int at = k < wide ? s_toff[e] + k : s_toff[p.E] + s_soff[e] + k - wide;
-      int32_t* tl = p.tiles + 4 + 4 * at;
-      tl[0] = e;
-      tl[1] = s_off[e] + k * p.tile_rows;
-      tl[2] = min(p.tile_rows, n - k * p.tile_rows);
-      tl[3] = 0;
+  // 4 threads per expert: its tiles k, k + 4, ...
+  for (int i = tid; i < 4 * p.E; i += 1024) {
+    const int e = i >> 2;
+    const int n = sm.cnt[e];
+    const int wide = tiles_of(p, n) - narrow_of(p, n);
+    for (int k = i & 3; k * p.tile_rows < n; k += 4) {
+      const int at = k < wide ? sm.toff[e] + k : sm.toff[p.E] + sm.soff[e] + k - wide;
+      *reinterpret_cast<int4*>(p.tiles + 4 + 4 * at) =
+          make_int4(e, sm.off[e] + k * p.tile_rows, min(p.tile_rows, n - k * p.tile_rows), 0);
     }
   }
 }
 
+// One work-group per work-group of fm_route_kernel, placing that one's pairs.
+// Each adds up the counts of all (they are few: 256 x E at most) for the
+// experts' totals and, over the work-groups before it, its own offsets; the
+// first also writes the tile table. Against one work-group that counted all
+// pairs by LDS atomics: M = 4001, E = 64, topk = 6 21 -> 5 us, M = 4096, E = 8,
+// topk = 2 8.5 -> 4.9 us (rocprof).
 __global__ void __launch_bounds__(1024) fm_plan_kernel(const PlanParams p) {
   __shared__ PlanSmem sm;
-  plan_body(p, sm);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int b = blockIdx.x;
+  // this work-group's first pairs, loaded ahead of the counts
+  const int64_t i0 = int64_t(b) * p.pairs_per_wg;
+  const int64_t i1 = i0 + p.pairs_per_wg < p.P ? i0 + p.pairs_per_wg : p.P;
+  const int32_t first = i0 + tid < i1 ? p.ids[i0 + tid] : 0;
+  for (int e = tid; e < kMaxExperts; e += 1024) {
+    sm.cnt[e] = 0;
+    sm.cur[e] = 0;
+  }
+  __syncthreads();
+  // thread (g, e): the work-groups g, g + G, ... of expert e
+  const int le = p.E <= 1 ? 0 : 32 - __builtin_clz(p.E - 1);  // log2 of E, rounded up
+  const int e = tid & ((1 << le) - 1);
+  int tot = 0, pre = 0;
+  if (e < p.E) {
+    const int step = 1024 >> le;
+    for (int w0 = tid >> le; w0 < p.wgs; w0 += 16 * step) {
+      int v[16];  // all loads of a batch in flight
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int w = w0 + j * step;
+        v[j] = w < p.wgs ? p.hist[w * p.E + e] : 0;
+      }
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        tot += v[j];
+        pre += w0 + j * step < b ? v[j] : 0;
+      }
+    }
+  }
+  for (int o = 1 << le; o < 64; o <<= 1) {
+    tot += __shfl_xor(tot, o);
+    pre += __shfl_xor(pre, o);
+  }
+  if (e < p.E && lane >> le == 0) {
+    atomicAdd(&sm.cnt[e], tot);
+    atomicAdd(&sm.cur[e], pre);
+  }
+  __syncthreads();
+  if (tid < 64) plan_scan(p, sm);
+  __syncthreads();
+  auto place = [&](int64_t i, int32_t id) {
+    const int x = id & 255;
+    p.sorted[sm.off[x] + sm.cur[x] + (id >> 8)] = int32_t(i);
+  };
+  if (i0 + tid < i1) place(i0 + tid, first);
+  for (int64_t i = i0 + tid + 1024; i < i1; i += 1024) place(i, p.ids[i]);
+  if (b == 0) plan_tiles(p, sm);
 }
 
-// Few tokens (decode): routing and plan in one work-group, one launch fewer.
-// Wave w routes token w. (With 4 tokens per wave, at M = 64, the one
-// work-group took 18.5 us against 6.5 + 6.5 for the two launches.)
-constexpr int kFusedRouteTokens = 16;
+// Few tokens (decode): routing and plan in one work-group, one launch fewer,
+// the ids kept in LDS. Wave w routes token w. M = 1, E = 8, topk = 2: 5.6 ->
+// 3.8 us with the DPP argmax and without the ids' way through memory.
+template <int kPer>
 __global__ void __launch_bounds__(1024) fm_route_plan_kernel(const RouteParams rp,
                                                              const PlanParams pp) {
   __shared__ PlanSmem sm;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  constexpr int kPerWave = kFusedRouteTokens / 16;
-  float raw[kPerWave][kPer];
-#pragma unroll
-  for (int j = 0; j < kPerWave; ++j) {
-    const int64_t t = wave + 16 * j;
-    if (t < rp.M) load_scores(rp, t, lane, raw[j]);
-  }
-#pragma unroll
-  for (int j = 0; j < kPerWave; ++j) {
-    const int64_t t = wave + 16 * j;
-    if (t < rp.M) {
-      route_token(rp, t, lane, raw[j]);
-      if (rp.zero_out != nullptr) clear_out_row(rp, t, lane);
-    }
-  }
-  // the ids and weights are in memory before any thread of the group reads
-  // them back (same CU: the workgroup barrier orders them once stored)
-  __builtin_amdgcn_s_waitcnt(0);
+  __shared__ int s_id[kFusedTokens * kMaxTopk];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  if (tid < kMaxExperts) sm.cnt[tid] = 0;
+  static_assert(kFusedTokens <= 16, "one token per wave");
+  float raw[kPer];
+  if (wave < rp.M) load_scores(rp, wave, lane, raw);
   __syncthreads();
-  plan_body(pp, sm);
+  if (wave < rp.M) {
+    route_token(rp, wave, lane, raw, [&](int slot, int e) {
+      s_id[wave * rp.topk + slot] = e | atomicAdd(&sm.cnt[e], 1) << 8;
+    });
+    if (rp.zero_out != nullptr) clear_out_row(rp, wave, lane);
+  }
+  __syncthreads();
+  if (tid < 64) plan_scan(pp, sm);
+  __syncthreads();
+  for (int i = tid; i < int(pp.P); i += 1024) {
+    const int id = s_id[i];
+    pp.sorted[sm.off[id & 255] + (id >> 8)] = i;
+  }
+  plan_tiles(pp, sm);
 }
 
 // ============================================================================
@@ -1337,7 +1413,7 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   uint8_t* ws = static_cast<uint8_t*>(a->workspace);
   int32_t* ids = reinterpret_cast<int32_t*>(ws + pl.ids_off);
   float* wts = reinterpret_cast<float*>(ws + pl.wts_off);
-  int32_t* eoff = reinterpret_cast<int32_t*>(ws + pl.eoff_off);
+  int32_t* hist = reinterpret_cast<int32_t*>(ws + pl.hist_off);
   int32_t* sorted = reinterpret_cast<int32_t*>(ws + pl.sorted_off);
   int32_t* tiles = reinterpret_cast<int32_t*>(ws + pl.tiles_off);
   __bf16* inter = reinterpret_cast<__bf16*>(ws + pl.inter_off);
@@ -1348,6 +1424,8 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   rp.s_score = a->s_score;
   rp.ids = ids;
   rp.wts = wts;
+  rp.hist = hist;
+  rp.tokens_per_wg = pl.tokens_per_wg;
   rp.M = a->M;
   rp.E = int(a->E);
   rp.topk = int(a->topk);
@@ -1365,22 +1443,29 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   }
   PlanParams pp{};
   pp.ids = ids;
-  pp.eoff = eoff;
+  pp.hist = hist;
+  pp.wgs = pl.route_wgs;
+  pp.pairs_per_wg = pl.tokens_per_wg * int(a->topk);
   pp.sorted = sorted;
   pp.tiles = tiles;
   pp.P = pl.P;
   pp.E = int(a->E);
   pp.tile_rows = pl.tile_rows;
   pp.narrow_rows = pl.narrow_rows;
-  if (a->M <= kFusedRouteTokens) {  // one launch, reported as the plan's
+  const bool e64 = a->E <= 64;
+  if (pl.route_wgs == 0) {  // one launch, reported as the plan's
     void* ka[] = {&rp, &pp};
-    if (!run(FM_KERNEL_PLAN, fn(fm_route_plan_kernel), dim3(1), dim3(1024), ka)) return FM_EHIP;
+    if (!run(FM_KERNEL_PLAN, e64 ? fn(fm_route_plan_kernel<1>) : fn(fm_route_plan_kernel<4>),
+             dim3(1), dim3(1024), ka))
+      return FM_EHIP;
   } else {
+    const dim3 grid(unsigned(pl.route_wgs));
     void* kr[] = {&rp};
-    if (!run(FM_KERNEL_ROUTE, fn(fm_route_kernel), dim3(unsigned((a->M + 3) / 4)), dim3(256), kr))
+    if (!run(FM_KERNEL_ROUTE, e64 ? fn(fm_route_kernel<1>) : fn(fm_route_kernel<4>), grid,
+             dim3(64 * kRouteWaves), kr))
       return FM_EHIP;
     void* kp[] = {&pp};
-    if (!run(FM_KERNEL_PLAN, fn(fm_plan_kernel), dim3(1), dim3(1024), kp)) return FM_EHIP;
+    if (!run(FM_KERNEL_PLAN, fn(fm_plan_kernel), grid, dim3(1024), kp)) return FM_EHIP;
   }
 
   GemmParams g1{};

@@ -177,6 +177,20 @@ def test_gemm_tiles_at_their_edges(gpu_sa, counts, K, N):
     check(out, fused_moe_ref(*cpu(hidden, w1, w2, score), 1), f"{counts[:6]}")
 
 
+@pytest.mark.parametrize("shape", [(16, 256, 128, 256, 32), (17, 256, 128, 65, 3),
+                                   (100, 256, 128, 256, 32), (4097, 256, 128, 9, 2),
+                                   (50, 256, 128, 1, 1)])
+def test_routing_over_work_groups(gpu_sa, shape):
+    """Routing and plan in one work-group and over several, the last one ragged
+    and with 16 or 32 tokens each, one and four experts per lane; half the
+    rows have integer scores (ties)."""
+    M, K, N, E, topk = shape
+    hidden, w1, w2, score = make_inputs(M, K, N, E, seed=14)
+    score[::2] = score[::2].round()
+    check(op(hidden, w1, w2, score, topk), fused_moe_ref(*cpu(hidden, w1, w2, score), topk),
+          f"{shape}")
+
+
 @pytest.mark.parametrize("M", [16, 64])
 def test_streamed_final_sum_forms(gpu_sa, M):
     """Streamed tiles where fm_gemm_kernel is the default: the atomic and the
