@@ -50,11 +50,11 @@
 //   sa_combine_kernel.
 // sa_fwd_wave_kernel  unsplit queries with topk <= 384 (per-query tiles of
 //   shared-row plans, or every query of a per-query plan): one wave64 work-
-//   group per two queries, a stream of 16-row steps through the wave's own
-//   2-deep LDS-DMA ring, no barrier. S^T = K . Q^T (16x16x32 MFMA, Q^T as
-//   an AGPR operand), the softmax inside the wave, O += P . V with
-//   v_mfma_f32_16x16x16_bf16 taking P from the S^T accumulators. Each
-//   query's rows are sorted ascending when a batch's kv exceeds an XCD's L2.
+//   group per query, eight per CU, 16-row steps through one LDS buffer, no
+//   barrier. S^T = K . Q^T (16x16x32 MFMA), the softmax inside the wave,
+//   O += P . V with v_mfma_f32_16x16x16_bf16 taking P from the S^T
+//   accumulators. Each query's rows are sorted ascending when a batch's kv
+//   exceeds an XCD's L2.
 // sa_combine_kernel  merges the topk parts of one (query, head), folds the
 //   sink and stores bf16.
 // sa_merge_kernel  merges caller-supplied (o, lse) partials (sa_merge).
@@ -1734,48 +1734,58 @@ __global__ void __launch_bounds__(kOrderThreads) sa_order_kernel(const OrderPara
 // per-query wave launch
 // ============================================================================
 // For short queries (topk <= kWaveMaxTopk, no split): one wave64 work-group
-// per kWQueries consecutive queries (of a per-query tile in a shared-row
-// plan, else of the flattened b x m), run as
-// one stream of kWRows-row steps through the wave's own 2-deep LDS ring, with
-// no barrier and no exchange with another wave. Per step:
+// per query (of a per-query tile in a shared-row plan, else of the flattened
+// b x m), in steps of kWRows rows, with no barrier and no exchange with
+// another wave. Per step:
 //  * S^T = K . Q^T with v_mfma_f32_16x16x32_bf16 (16 rows x 16 heads, K = d,
-//    Q^T resident in registers); the 16 gathers of the next step ride between
-//    its 16 MFMAs;
+//    Q^T resident in registers);
 //  * the online softmax of the 16 heads inside the wave (a head's 16 scores
 //    sit in 4 lanes x 4 values);
 //  * O += P . V with v_mfma_f32_16x16x16_bf16. The S^T accumulator layout
 //    (lane (head n, g) holds rows 4g..4g+3) is that MFMA's A operand layout,
 //    so P stays in registers; V comes from the same LDS rows by transposing
-//    reads.
-// Four work-groups fit in a CU's LDS, one per SIMD, and a CU takes the next
-// one as soon as one ends, so one wave's start and end overlap the others'
-// steps. The list holds 32-bit byte offsets of the rows in the query's batch
-// of kv (the host checks that they fit).
+//    reads;
+//  * the gathers of the next step, into the same buffer.
+// One buffer per wave (17 KiB) and 256 registers let eight work-groups share a
+// CU, two per SIMD: one computes while the other waits for its rows, and a CU
+// takes the next one as soon as one ends. (A two-deep ring per wave allowed
+// one wave per SIMD, bound by its own dependent chain.)
+// Bound: at topk 128 by HBM, q in and o out (462 us at the copy rate for 65 536
+// queries); measured 64 x 1024, kv_len 1024, topk 128, kernel 960 -> 713 us
+// (883 with the old stores), 16 x 4096, kv_len 4096 992 -> 768, 1 x 16384,
+// kv_len 16384 317 -> 262. Without its gathers 492, without its stores 548,
+// without both and Q's loads 314. Each 16 slots more cost 0.84 us per SIMD,
+// 1 750 cycles, of which the MFMAs of two waves are 1 540. Dealing whole
+// batches to the XCDs, or gathering between the last MFMAs, changed nothing.
+// The list holds 32-bit byte offsets of the rows in the query's batch of kv
+// (the host checks that they fit).
 constexpr int kWRows = 16;               // rows per step
 constexpr int kWPitch = kRowBytes + 48;  // LDS row pitch (bytes)
-constexpr int kWQueries = 2;             // queries per work-group
 constexpr int kWVAhead = 8;              // V fragments in flight in O += P . V
 // A batch's kv span (bytes) above which the wave kernel sorts each query's
 // rows: an XCD's L2 (4 MiB on MI355X)
 constexpr int64_t kWaveSortBytes = int64_t(4) << 20;
 constexpr int kWSlots = kWaveMaxTopk / 64;
-static_assert(kTQ % kWQueries == 0, "a tile's queries split evenly");
-static_assert(kWQueries == 2, "the cursor state is two queries' scalars");
-static_assert(kDim / 32 == kWRows, "one gather per S^T MFMA");
+static_assert(kDim / 32 == kWRows, "one row per S^T MFMA");
 
 struct WaveSmem {
-  uint8_t tile[2][kWRows * kWPitch];
-  int32_t list[kWQueries * kWaveMaxTopk];
+  uint8_t tile[kWRows * kWPitch];
+  int32_t list[kWaveMaxTopk];
 };
-static_assert(4 * sizeof(WaveSmem) <= 160 * 1024, "four work-groups per CU");
+static_assert(8 * sizeof(WaveSmem) <= 160 * 1024, "eight work-groups per CU");
 
 // Stores query (bi, mi)'s o (and lse) from the wave's state: lane (n, g)
-// holds O[head 4g + j][16 blk + n]. Lanes n and n ^ 1 swap half their values
-// (DPP), so that each store writes two adjacent columns of one head: the even
-// lane heads 4g and 4g + 1, the odd lane heads 4g + 2 and 4g + 3. Needs o and
-// its strides 4-byte aligned (validate() asks for 16 bytes).
-__device__ __forceinline__ void wave_epilogue(const FwdParams& p, int64_t bi, int64_t mi,
-                                              float m_run, float l_run, const f32x4 (&oacc)[32]) {
+// holds O[head 4g + j][16 blk + n]. The rows go through the LDS tile (`rows`,
+// free by now), so that every global store writes one head's whole 1 KiB row:
+// stores of 4 bytes per lane straight from the accumulators reach HBM as
+// partial lines (64 x 1024 queries, topk 128: 335 us of a 884 us launch).
+// Lanes n and n ^ 1 first swap half their values (DPP), so that each LDS write
+// holds two adjacent columns of one head: the even lane heads 4g and 4g + 1,
+// the odd lane heads 4g + 2 and 4g + 3. At the 1072-byte pitch a write hits
+// every bank once.
+__device__ __forceinline__ void wave_epilogue(const FwdParams& p, uint8_t* rows, int64_t bi,
+                                              int64_t mi, float m_run, float l_run,
+                                              const f32x4 (&oacc)[32]) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63;
@@ -1789,9 +1799,8 @@ __device__ __forceinline__ void wave_epilogue(const FwdParams& p, int64_t bi, in
 #pragma unroll
   for (int j = 0; j < 4; ++j) fj[j] = __shfl(f, 4 * g + j);
   const bool odd = (n & 1) != 0;
-  __bf16* const r0 =
-      p.o + bi * p.so_b + mi * p.so_m + int64_t(4 * g + (odd ? 2 : 0)) * p.so_h + (n & ~1);
-  __bf16* const r1 = r0 + p.so_h;
+  uint8_t* const r0 = rows + (4 * g + (odd ? 2 : 0)) * kWPitch + 2 * (n & ~1);
+  uint8_t* const r1 = r0 + kWPitch;
   auto swap = [](float x) {  // the value of lane n ^ 1
     return __builtin_bit_cast(
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
@@ -1804,290 +1813,193 @@ __device__ __forceinline__ void wave_epilogue(const FwdParams& p, int64_t bi, in
     const float x1 = swap(odd ? v1 : v3);
     const f32x2 a = odd ? f32x2{x0, v2} : f32x2{v0, x0};
     const f32x2 b = odd ? f32x2{x1, v3} : f32x2{v1, x1};
-    const bf16x2 ha = __builtin_convertvector(a, bf16x2);
-    const bf16x2 hb = __builtin_convertvector(b, bf16x2);
-    __builtin_nontemporal_store(__builtin_bit_cast(uint32_t, ha),
-                                reinterpret_cast<uint32_t*>(r0 + 16 * blk));
-    __builtin_nontemporal_store(__builtin_bit_cast(uint32_t, hb),
-                                reinterpret_cast<uint32_t*>(r1 + 16 * blk));
+    *reinterpret_cast<bf16x2*>(r0 + 32 * blk) = __builtin_convertvector(a, bf16x2);
+    *reinterpret_cast<bf16x2*>(r1 + 32 * blk) = __builtin_convertvector(b, bf16x2);
+  }
+  asm volatile("" ::: "memory");  // one wave: its LDS operations run in order
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  __bf16* const orow = p.o + bi * p.so_b + mi * p.so_m + 8 * lane;
+#pragma unroll
+  for (int h = 0; h < kHeads; ++h) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(rows + h * kWPitch + 16 * lane);
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(orow + int64_t(h) * p.so_h));
   }
 }
 
-// In a shared-row plan (FwdParams::meta set) work-group i runs queries
-// kWQueries * (i % parts) .. of tile i / parts (parts = kTQ / kWQueries) when
-// the index kernel made that tile per query; else queries kWQueries * i .. of
-// the p.nblocks queries of b x m (two of them may be in different batches).
-__global__ void __launch_bounds__(64, 1) sa_fwd_wave_kernel(const FwdParams p) {
+// In a shared-row plan (FwdParams::meta set) work-group i runs query i % kTQ
+// of tile i / kTQ when the index kernel made that tile per query; else query i
+// of the p.nblocks queries of b x m.
+__global__ void __launch_bounds__(64, 2) sa_fwd_wave_kernel(const FwdParams p) {
   __shared__ __attribute__((aligned(16))) WaveSmem sm;
-  constexpr int kParts = kTQ / kWQueries;
   const int lane = threadIdx.x;
   const int n = lane & 15;
   const int g = lane >> 4;
-  int64_t q0;  // the first query, as b * m + m
-  int nq;
+  int64_t bi, mi;
   if (p.meta != nullptr) {
-    const int64_t t = blockIdx.x / kParts;
-    const int64_t m0 = (t % p.tiles_per_b) * kTQ + (blockIdx.x % kParts) * kWQueries;
+    const int64_t t = blockIdx.x / kTQ;
+    bi = t / p.tiles_per_b;
+    mi = (t % p.tiles_per_b) * kTQ + blockIdx.x % kTQ;
+    if (mi >= p.m) return;
     if (__builtin_amdgcn_readfirstlane(p.meta[t * kMetaInts + 1]) == kModeShared) return;
-    nq = int(min(int64_t(kWQueries), p.m - m0));
-    q0 = (t / p.tiles_per_b) * p.m + m0;
   } else {
-    q0 = int64_t(blockIdx.x) * kWQueries;
-    nq = int(min(int64_t(kWQueries), p.nblocks - q0));
+    bi = blockIdx.x / p.m;
+    mi = blockIdx.x - bi * p.m;
   }
-  if (nq <= 0) return;
-  // batch and query of the two queries, as scalars (small arrays indexed by a
-  // loop variable end up in LDS, and what is read from there is not known
-  // to be uniform)
-  const int64_t qb0 = q0 / p.m, qm0 = q0 - qb0 * p.m;
-  const int64_t q1 = q0 + (nq > 1 ? 1 : 0);
-  const int64_t qb1 = q1 / p.m, qm1 = q1 - qb1 * p.m;
-  auto qb_of = [&](int j) { return j == 0 ? qb0 : qb1; };
-  auto qm_of = [&](int j) { return j == 0 ? qm0 : qm1; };
-  auto kv_of = [&](int j) {
-    return reinterpret_cast<const uint8_t*>(p.kv + qb_of(j) * p.skv_b);
-  };
   const int topk = int(p.topk);
   const uint32_t row_bytes = uint32_t(p.skv_n * 2);
 
-  // ---- indices, then query 0's Q^T (B operand: lane (n, g) holds head n,
-  // d = 32s + 8g .. +7 for k-step s) ----------------------------------------------
-  int raw[kWQueries][kWSlots];
+  // ---- indices, then Q^T (B operand: lane (n, g) holds head n, d = 32s + 8g
+  // .. +7 for k-step s) --------------------------------------------------------------
+  const int32_t* irow = p.idx + bi * p.si_b + mi * p.si_m;
+  int raw[kWSlots];
 #pragma unroll
-  for (int j = 0; j < kWQueries; ++j)
-#pragma unroll
-    for (int i = 0; i < kWSlots; ++i) {
-      const int sl = 64 * i + lane;
-      raw[j][i] = (j < nq && sl < topk) ? p.idx[qb_of(j) * p.si_b + qm_of(j) * p.si_m + sl] : -1;
-    }
+  for (int i = 0; i < kWSlots; ++i) raw[i] = 64 * i + lane < topk ? irow[64 * i + lane] : -1;
   bf16x8 qf[kDim / 32];
-  auto load_q = [&](int j) {
-    const __bf16* qrow =
-        p.q + qb_of(j) * p.sq_b + qm_of(j) * p.sq_m + int64_t(n) * p.sq_h + 8 * g;
+  const __bf16* qrow = p.q + bi * p.sq_b + mi * p.sq_m + int64_t(n) * p.sq_h + 8 * g;
 #pragma unroll
-    for (int s = 0; s < kDim / 32; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s);
-  };
-  // Q^T as the B operand of S^T lives in AGPRs: qa is written from qf once
-  // per query (the tied asm operand makes the compiler copy qf into the
-  // AGPRs there), and the MFMAs read it with an "a" constraint. Read straight
-  // from qf, the MFMAs made the compiler copy Q^T into AGPRs at every step
-  // (64 v_accvgpr_write per step), since qf changes inside the step loop when
-  // the next query's Q^T is loaded.
-  bf16x8 qa[kDim / 32];
-  auto q_to_agpr = [&]() {
-#pragma unroll
-    for (int s = 0; s < kDim / 32; ++s) asm volatile("" : "=a"(qa[s]) : "0"(qf[s]));
-  };
-  load_q(0);
+  for (int s = 0; s < kDim / 32; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s);
 
-  // ---- compaction: query j's valid slots at list[qsel(j) .. qsel(j + 1)) ----------
+  // ---- compaction of the valid slots ------------------------------------------------
   const unsigned long long below = (1ull << lane) - 1ull;
-  int pos = 0, qs1 = 0;
+  int cnt = 0;
   bool bad = false;
 #pragma unroll
-  for (int j = 0; j < kWQueries; ++j) {
-    if (j == 1) qs1 = pos;
-#pragma unroll
-    for (int i = 0; i < kWSlots; ++i) {
-      const int v = raw[j][i];
-      const bool ok = (v >= 0) && (int64_t(v) < p.kv_len);
-      bad |= (!ok && v != -1);
-      const unsigned long long bm = __ballot(ok);
-      if (ok) sm.list[pos + __popcll(bm & below)] = int32_t(uint32_t(v) * row_bytes);
-      pos += __popcll(bm);
-    }
+  for (int i = 0; i < kWSlots; ++i) {
+    const int v = raw[i];
+    const bool ok = (v >= 0) && (int64_t(v) < p.kv_len);
+    bad |= (!ok && v != -1);
+    const unsigned long long bm = __ballot(ok);
+    if (ok) sm.list[cnt + __popcll(bm & below)] = int32_t(uint32_t(v) * row_bytes);
+    cnt += __popcll(bm);
   }
-  const int qs2 = pos;
   if (bad && p.err != nullptr) flag_bad_index(p.err);
   __syncthreads();  // the list is written before it is read
-  auto qsel = [&](int j) { return j <= 0 ? 0 : j == 1 ? qs1 : qs2; };
-  auto nst = [&](int j) { return (qsel(j + 1) - qsel(j) + kWRows - 1) / kWRows; };
-  int total = 0;
-#pragma unroll
-  for (int j = 0; j < kWQueries; ++j) total += nst(j);
-  // Q^T and the indices complete before the first gather is issued, so that
-  // every later vmcnt(0) waits for the ring (and a Q^T issued after a gather)
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   if (p.sort_wave) {
     // Each query walks its rows in ascending order: the queries resident on
     // an XCD then sweep their batch's kv together, and a row that several of
     // them name is fetched into the XCD's L2 once. The sorted sequence does
     // not depend on the input order.
-    auto sort_query = [&](int j) {
-      uint32_t* s = reinterpret_cast<uint32_t*>(&sm.list[qsel(j)]);
-      const int n = qsel(j + 1) - qsel(j);
-      if (n <= 64)
-        sort_list_wave<1>(s, n);
-      else if (n <= 128)
-        sort_list_wave<2>(s, n);
-      else if (n <= 256)
-        sort_list_wave<4>(s, n);
-      else
-        sort_list_wave<8>(s, n);
-    };
+    uint32_t* s = reinterpret_cast<uint32_t*>(sm.list);
+    if (cnt <= 64)
+      sort_list_wave<1>(s, cnt);
+    else if (cnt <= 128)
+      sort_list_wave<2>(s, cnt);
+    else if (cnt <= 256)
+      sort_list_wave<4>(s, cnt);
+    else
+      sort_list_wave<8>(s, cnt);
     static_assert(kWaveMaxTopk <= 64 * 8, "the sort covers a query's slots");
-    sort_query(0);
-    if (nq > 1) sort_query(1);
   }
+  const int ns = (cnt + kWRows - 1) / kWRows;
 
-  // ---- the step stream ------------------------------------------------------------
-  // The issue cursor (ji, si): query and step of the next step to gather. Lane
-  // n < 16 holds the entry of the step's row n; entries past a query's last
-  // valid one take its first entry's row, whose scores are masked.
-  const uint32_t lds_rows = __builtin_amdgcn_readfirstlane(
-      uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)&sm.tile[0][0])));
-  int ji = 0, si = 0;
-  while (ji < kWQueries && nst(ji) == 0) ++ji;
-  // the rows' entries for the cursor's step; kvg = the base of their batch
-  const uint8_t* kvg = nullptr;
-  auto cursor_rows = [&]() {
-    const int e0 = qsel(ji);
-    const int e = e0 + si * kWRows + n;
-    const int rv = sm.list[e < qsel(ji + 1) ? e : e0];
-    kvg = kv_of(ji);
-    if (++si == nst(ji)) {
-      si = 0;
-      do {
-        ++ji;
-      } while (ji < kWQueries && nst(ji) == 0);
-    }
-    return rv;
+  // ---- steps ---------------------------------------------------------------------------
+  const uint32_t lds_rows =
+      __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)sm.tile)));
+  const uint8_t* kvb = reinterpret_cast<const uint8_t*>(p.kv + bi * p.skv_b);
+  // Lane n < 16 holds the entry of step s's row n; entries past the last valid
+  // one take the first entry's row, whose scores are masked.
+  auto step_rows = [&](int s) {
+    const int e = s * kWRows + n;
+    return sm.list[e < cnt ? e : 0];
   };
-  // kvg as a scalar (for the gathers' scalar base). readfirstlane returns
-  // int: each half goes through uint32_t so the low one is not sign-extended.
-  auto kv_scalar = [&]() {
-    const uint64_t a = reinterpret_cast<uint64_t>(kvg);
-    const uint32_t lo = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(a))));
-    const uint32_t hi = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(a >> 32))));
-    return reinterpret_cast<const uint8_t*>(uint64_t(lo) | uint64_t(hi) << 32);
+  auto gather = [&](int rv, int i) {
+    const uint32_t off = uint32_t(__builtin_amdgcn_readlane(rv, i));
+    lds_dma_row(kvb + off, 16 * lane, lds_rows + uint32_t(i * kWPitch));
   };
-  if (total > 0) {
-    const int rv = cursor_rows();
-    const uint8_t* kvs = kv_scalar();
+  if (ns > 0) {
+    const int rv = step_rows(0);
 #pragma unroll
-    for (int i = 0; i < kWRows; ++i) {
-      const uint32_t off = uint32_t(__builtin_amdgcn_readlane(rv, i));
-      lds_dma_row(kvs + off, 16 * lane, lds_rows + uint32_t(i * kWPitch));
-    }
+    for (int i = 0; i < kWRows; ++i) gather(rv, i);
   }
 
   f32x4 oacc[32];
   float m_run = -INFINITY, l_run = 0.f;
 #pragma unroll
   for (int blk = 0; blk < 32; ++blk) oacc[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int gstep = 0;
-  int qloaded = 0;  // the query whose Q^T is in qf
-  for (int j = 0; j < nq; ++j) {
-    const int ns = nst(j);
-    int jn = j + 1;  // the next query with a valid slot
-    while (jn < nq && nst(jn) == 0) ++jn;
-    if (ns > 0 && qloaded != j) {  // only after a query without a valid slot
-      load_q(j);
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-      qloaded = j;
-    }
-    for (int s = 0; s < ns; ++s, ++gstep) {
-      // this step's rows (and a Q^T issued during the last step) have landed,
-      // and the reads of the buffer the next gathers fill are complete
-      __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-      asm volatile("" ::: "memory");
-      if (s == 0) q_to_agpr();  // this query's Q^T, landed
-      const bool dma = gstep + 1 < total;
-      const int rv = dma ? cursor_rows() : 0;
-      const uint8_t* kvs = kv_scalar();
-      const uint32_t lnext = lds_rows + uint32_t(((gstep + 1) & 1) * kWRows * kWPitch);
-      const uint8_t* tb = sm.tile[gstep & 1];
-      const int nrows = qsel(j + 1) - qsel(j) - s * kWRows;
+  const uint8_t* krow = sm.tile + n * kWPitch + 16 * g;
+  const uint8_t* vb = sm.tile + (4 * g + (n >> 2)) * kWPitch + 8 * (n & 3);
+  for (int s = 0; s < ns; ++s) {
+    const int rv = s + 1 < ns ? step_rows(s + 1) : 0;
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this step's rows have landed
+    asm volatile("" ::: "memory");
+    const int nrows = cnt - s * kWRows;
 
-      // S^T for the step's 16 rows (A: lane (row n, g) reads d = 32s + 8g ..);
-      // two accumulator chains, K fragments read 3 MFMAs ahead
-      f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-      const uint8_t* krow = tb + n * kWPitch + 16 * g;
-      auto s_chain = [&](auto with_dma) {
-        bf16x8 kf[4];
+    // S^T for the step's 16 rows (A: lane (row n, g) reads d = 32s + 8g ..);
+    // two accumulator chains, K fragments read 3 MFMAs ahead
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    bf16x8 kf[4];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) kf[k] = *reinterpret_cast<const bf16x8*>(krow + 64 * k);
+    for (int k = 0; k < 3; ++k) kf[k] = *reinterpret_cast<const bf16x8*>(krow + 64 * k);
 #pragma unroll
-        for (int k = 0; k < kDim / 32; ++k) {
-          if (k + 3 < kDim / 32)
-            kf[(k + 3) & 3] = *reinterpret_cast<const bf16x8*>(krow + 64 * (k + 3));
-          if (k & 1)
-            mfma32_bagpr(sb, kf[k & 3], qa[k]);
-          else
-            mfma32_bagpr(sa, kf[k & 3], qa[k]);
-          if constexpr (decltype(with_dma)::value) {
-            const uint32_t off = uint32_t(__builtin_amdgcn_readlane(rv, k));
-            lds_dma_row(kvs + off, 16 * lane, lnext + uint32_t(k * kWPitch));
-          }
-          __builtin_amdgcn_sched_barrier(0);  // keep the interleave
-        }
-      };
-      if (dma)
-        s_chain(std::true_type{});
+    for (int k = 0; k < kDim / 32; ++k) {
+      if (k + 3 < kDim / 32)
+        kf[(k + 3) & 3] = *reinterpret_cast<const bf16x8*>(krow + 64 * (k + 3));
+      if (k & 1)
+        sb = mfma_16x16x32(kf[k & 3], qf[k], sb);
       else
-        s_chain(std::false_type{});
-      // The first V fragments of O += P . V (they do not depend on P) are
-      // read now, so that their LDS latency passes under the softmax: lane
-      // (n, g) reads V[rows 4g .. 4g + 3][16 blk + n] of column block blk.
-      const uint8_t* vb = tb + (4 * g + (n >> 2)) * kWPitch + 8 * (n & 3);
-      bf16x4 vf[kWVAhead];
-#pragma unroll
-      for (int i = 0; i < kWVAhead; ++i) vf[i] = lds_read_tr16(vb + 32 * i);
-      mfma_agpr_drain();  // S^T is read by VALU below
-      if (s == ns - 1 && jn < nq) load_q(jn);  // Q^T is no longer read
-
-      // online softmax: lane (n, g) holds S[head n][row 4g + j]
-      float sv[4];
-      float mx = -INFINITY;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        sv[k] = (4 * g + k < nrows) ? (sa[k] + sb[k]) * p.scale_log2 : -INFINITY;
-        mx = fmaxf(mx, sv[k]);
-      }
-      mx = wave_max16(mx);  // finite: the step's row 0 is valid
-      float alpha = 1.f;
-      if (mx > m_run + kRescaleLog2) {
-        // (O, l still 0 at first; v_exp_f32 as in the per-query step)
-        alpha = m_run == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mx);
-        m_run = mx;
-      }
-      float psum = 0.f;
-      bf16x4 pb;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float pk = __builtin_amdgcn_exp2f(sv[k] - m_run);
-        psum += pk;
-        pb[k] = static_cast<__bf16>(pk);
-      }
-      l_run = l_run * alpha + psum;
-      if (__any(alpha != 1.f)) {
-        float ak[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) ak[k] = __shfl(alpha, 4 * g + k);
-#pragma unroll
-        for (int blk = 0; blk < 32; ++blk)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) oacc[blk][k] *= ak[k];
-      }
-
-      // O += P . V over the 32 column blocks, each V fragment read kWVAhead
-      // MFMAs ahead of its own (the MFMA takes 16 cycles, an LDS read about
-      // 100: left to itself the compiler read 3 ahead and each MFMA waited)
-#pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        const bf16x4 v = vf[i % kWVAhead];
-        if (i + kWVAhead < 32) vf[i % kWVAhead] = lds_read_tr16(vb + 32 * (i + kWVAhead));
-        oacc[i] = mfma_16x16x16(pb, v, oacc[i]);
-        __builtin_amdgcn_sched_barrier(0);  // keep the interleave
-      }
+        sa = mfma_16x16x32(kf[k & 3], qf[k], sa);
+      __builtin_amdgcn_sched_barrier(0);  // keep the interleave
     }
-    if (ns > 0 && jn < nq) qloaded = jn;
-    wave_epilogue(p, qb_of(j), qm_of(j), m_run, l_run, oacc);
-    m_run = -INFINITY;
-    l_run = 0.f;
+    // The first V fragments of O += P . V (they do not depend on P) are read
+    // now, so that their LDS latency passes under the softmax: lane (n, g)
+    // reads V[rows 4g .. 4g + 3][16 blk + n] of column block blk.
+    bf16x4 vf[kWVAhead];
 #pragma unroll
-    for (int blk = 0; blk < 32; ++blk) oacc[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < kWVAhead; ++i) vf[i] = lds_read_tr16(vb + 32 * i);
+
+    // online softmax: lane (n, g) holds S[head n][row 4g + j]
+    float sv[4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      sv[k] = (4 * g + k < nrows) ? (sa[k] + sb[k]) * p.scale_log2 : -INFINITY;
+      mx = fmaxf(mx, sv[k]);
+    }
+    mx = wave_max16(mx);  // finite: the step's row 0 is valid
+    float alpha = 1.f;
+    if (mx > m_run + kRescaleLog2) {
+      // (O, l still 0 at first; v_exp_f32 as in the per-query step)
+      alpha = m_run == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mx);
+      m_run = mx;
+    }
+    float psum = 0.f;
+    bf16x4 pb;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float pk = __builtin_amdgcn_exp2f(sv[k] - m_run);
+      psum += pk;
+      pb[k] = static_cast<__bf16>(pk);
+    }
+    l_run = l_run * alpha + psum;
+    if (__any(alpha != 1.f)) {
+      float ak[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ak[k] = __shfl(alpha, 4 * g + k);
+#pragma unroll
+      for (int blk = 0; blk < 32; ++blk)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) oacc[blk][k] *= ak[k];
+    }
+
+    // O += P . V over the 32 column blocks, each V fragment read kWVAhead
+    // MFMAs ahead of its own (the MFMA takes 16 cycles, an LDS read about
+    // 100: left to itself the compiler read 3 ahead and each MFMA waited)
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const bf16x4 v = vf[i % kWVAhead];
+      if (i + kWVAhead < 32) vf[i % kWVAhead] = lds_read_tr16(vb + 32 * (i + kWVAhead));
+      oacc[i] = mfma_16x16x16(pb, v, oacc[i]);
+      __builtin_amdgcn_sched_barrier(0);  // keep the interleave
+    }
+    // every read of the buffer is complete: the next step's rows go into it
+    if (s + 1 < ns) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < kWRows; ++i) gather(rv, i);
+    }
   }
+  wave_epilogue(p, sm.tile, bi, mi, m_run, l_run, oacc);
 }
 
 // ============================================================================
@@ -3126,7 +3038,7 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
   auto launch_query = [&]() -> int {
     if (p.meta == nullptr && wave_ok)
       return run(SA_KERNEL_WAVE, fn(sa_fwd_wave_kernel),
-                 dim3(unsigned((p.nblocks + kWQueries - 1) / kWQueries)), dim3(64), 0, &p);
+                 dim3(unsigned(p.nblocks)), dim3(64), 0, &p);
     const dim3 grid(unsigned(p.nblocks)), block(kThreads);
     const bool two = p.nblocks >= 2 * int64_t(cus);
     const void* k = p.meta != nullptr
@@ -3221,7 +3133,7 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
         p.ord.order = nullptr;
       }
       const int wrc = run(SA_KERNEL_WAVE, fn(sa_fwd_wave_kernel),
-                          dim3(unsigned(plan.ntiles * (kTQ / kWQueries))), dim3(64), 0, &p);
+                          dim3(unsigned(plan.ntiles * kTQ)), dim3(64), 0, &p);
       if (wrc != SA_OK) return wrc;
     } else {
       p.nblocks = plan.ntiles + (p.ord.order != nullptr ? 1 : 0);
