@@ -119,6 +119,20 @@ constexpr int64_t kSharedTileNs = 10000;
 constexpr int64_t kSharedPairNs10 = 66;   // x 10
 constexpr int64_t kQueryUnitNs = 2100;
 constexpr int64_t kQuerySlotNs = 27;
+// Queries of topk <= kWaveMaxTopk run one wave each: 1 350 plus 12 per slot (64
+// x 1024 queries, kv_len 1 024 and 1 280, topk 128, 200 and 384), or 22 where
+// a batch's kv exceeds an XCD's L2 (topk 128 at 16 384, 300 at 20 480). Whole
+// calls, tiles shared -> per query: 64 x 1024, kv_len 1 280, topk 384 2 377 ->
+// 1 511 us; 64 x 512, 512, 128 578 -> 381; 64 x 1024, 600, 256 1 411 -> 1 144;
+// causal 4 096, topk 256 122 -> 100. The pair-skipping form of the shared tiles
+// (kTQ * topk < kv_len) costs about 4.5 per pair where queries share windows
+// of rows; priced at 6.6 against the wave's figures, such tiles went per query
+// too early: 4 x 4096, kv_len 8 192, topk 256 470 -> 514 us; 2 x 2000, 16 384,
+// 320 186 -> 222.
+constexpr int64_t kWaveUnitNs = 1350;
+constexpr int64_t kWaveSlotNs = 12;
+constexpr int64_t kWaveFarSlotNs = 22;
+constexpr int64_t kSharedSkipPairNs10 = 45;
 constexpr int64_t kPlacedQueryUnitNs = 4900;
 constexpr int64_t kPlacedQuerySlotNs = 35;
 constexpr int64_t kSharedMarginPct = 85;  // shared only below 85 % of per-query
@@ -126,11 +140,10 @@ constexpr int64_t kSharedMarginPct = 85;  // shared only below 85 % of per-query
 // The mode rule: shared when the tile's shared-row time is below
 // kSharedMarginPct % of its queries' per-query time.
 __host__ __device__ constexpr bool shared_is_cheaper(int64_t n_union, int64_t n_valid,
-                                                    int64_t queries, bool placed_regime) {
-  return 100 * (10 * kSharedTileNs + kSharedPairNs10 * kTQ * n_union) <=
-         kSharedMarginPct * 10 *
-             ((placed_regime ? kPlacedQueryUnitNs : kQueryUnitNs) * queries +
-              (placed_regime ? kPlacedQuerySlotNs : kQuerySlotNs) * n_valid);
+                                                    int64_t queries, int64_t pair_ns10,
+                                                    int64_t unit_ns, int64_t slot_ns) {
+  return 100 * (10 * kSharedTileNs + pair_ns10 * kTQ * n_union) <=
+         kSharedMarginPct * 10 * (unit_ns * queries + slot_ns * n_valid);
 }
 
 // An order entry of the tile order kernel is (key << kOrderTileBits) | tile:
@@ -202,7 +215,9 @@ struct IndexParams {
   int64_t tiles_per_b, cap;
   int force;            // shared mode whenever the counts fit
   int vec4;             // indices readable as int4 (aligned base, strides and topk)
-  int placed_regime;    // every tile starts at once (see kPlacedQueryUnitNs)
+  // the mode rule's prices: of a shared (query, row) pair (x 10), of a per-query
+  // query and of its slot
+  int pair_ns10, unit_ns, slot_ns;
 };
 
 struct TileParams {
@@ -1231,7 +1246,7 @@ __global__ void __launch_bounds__(kIdxThreads) sa_tile_index_kernel(const IndexP
     if (lane == 0 && nfresh != 0) atomicAdd(&s_nunion, nfresh);
     __syncthreads();
     // the first setter of each row's bit counted it: s_nunion is the union size
-    const bool cheaper = shared_is_cheaper(s_nunion, s_nvalid, qt, p.placed_regime != 0);
+    const bool cheaper = shared_is_cheaper(s_nunion, s_nvalid, qt, p.pair_ns10, p.unit_ns, p.slot_ns);
     if (p.force == 0 && !cheaper) {
       if (tid == 0) {
         int32_t* meta = p.meta + tile * kMetaInts;
@@ -1312,7 +1327,7 @@ __global__ void __launch_bounds__(kIdxThreads) sa_tile_index_kernel(const IndexP
     // are serialised), so s_nunion is the union size, and the mode can be
     // decided now: a per-query tile needs no union, so its scan and write are
     // skipped. (A count carry can only make a tile per query, below.)
-    const bool cheaper = shared_is_cheaper(s_nunion, s_nvalid, qt, p.placed_regime != 0);
+    const bool cheaper = shared_is_cheaper(s_nunion, s_nvalid, qt, p.pair_ns10, p.unit_ns, p.slot_ns);
     if (p.force == 0 && !cheaper) {
       if (tid == 0) {
         int32_t* meta = p.meta + tile * kMetaInts;
@@ -3066,7 +3081,15 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
     ip.vec4 = ((reinterpret_cast<uintptr_t>(a->idx) & 15u) == 0 && a->topk % 4 == 0 &&
                a->sidx[0] % 4 == 0 && a->sidx[1] % 4 == 0) ? 1 : 0;
     // from the shape alone, so that an index plan makes the plain call's modes
-    ip.placed_regime = (2 * plan.ntiles >= cus && plan.ntiles <= cus) ? 1 : 0;
+    const bool placed_regime = 2 * plan.ntiles >= cus && plan.ntiles <= cus;
+    const bool waves = a->topk <= kWaveMaxTopk;  // one wave per query
+    ip.pair_ns10 = int(waves && !placed_regime && kTQ * a->topk < a->kv_len ? kSharedSkipPairNs10
+                                                                           : kSharedPairNs10);
+    ip.unit_ns = int(placed_regime ? kPlacedQueryUnitNs : waves ? kWaveUnitNs : kQueryUnitNs);
+    ip.slot_ns = int(placed_regime ? kPlacedQuerySlotNs
+                     : !waves      ? kQuerySlotNs
+                     : p.sort_wave ? kWaveFarSlotNs
+                                   : kWaveSlotNs);
     int32_t* order = reinterpret_cast<int32_t*>(ws + plan.order_off);
     const bool planned = what == Launch::kCall && (a->flags & SA_FLAG_PLANNED) != 0;
     // Between half as many tiles as CUs and as many, every tile starts at
@@ -3074,7 +3097,7 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
     // itself and no order is made. (Fewer tiles keep the order: with a CU or
     // more per tile, the longest-first order beats XCD placement. An index
     // plan always holds an order.)
-    const bool placed = what == Launch::kCall && !planned && ip.placed_regime != 0;
+    const bool placed = what == Launch::kCall && !planned && placed_regime;
     if (!planned) {
       const size_t lds = size_t(a->kv_len) * sizeof(unsigned long long);
       // long caches (one work-group per CU by LDS): twice the threads, half
