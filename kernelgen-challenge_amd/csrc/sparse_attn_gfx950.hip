@@ -55,6 +55,10 @@
 //   O += P . V with v_mfma_f32_16x16x16_bf16 taking P from the S^T
 //   accumulators. Each query's rows are sorted ascending when a batch's kv
 //   exceeds an XCD's L2.
+// sa_fwd_waves_kernel  unsplit queries of 385 to 2 048 slots over caches too
+//   long for shared tiles: W = 1, 2 or 4 waves per query, each running every
+//   W-th step of the query's sorted rows as the wave kernel does, merged at
+//   the end through LDS.
 // sa_combine_kernel  merges the topk parts of one (query, head), folds the
 //   sink and stores bf16.
 // sa_merge_kernel  merges caller-supplied (o, lse) partials (sa_merge).
@@ -65,6 +69,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <limits>
 #include <type_traits>
 
 #include "sa_plan.h"
@@ -675,9 +680,9 @@ __device__ __forceinline__ void query_epilogue(const FwdParams& p, QuerySmemT<kR
   }
 }
 
-// Sorts the first kThreads * R entries of the LDS list `s` ascending, in
-// place: a bitonic network over kThreads * R keys, R consecutive keys per
-// thread. Entries at or past `n` count as +inf, so the n valid entries end up
+// Sorts the first NT * R entries of the LDS list `s` ascending, in place, with
+// a work-group of NT threads: a bitonic network over NT * R keys, R consecutive
+// keys per thread. Entries at or past `n` count as the largest T, so the n valid entries end up
 // in front, sorted; the caller reads no further. Steps whose partner key is
 // in the same thread compare registers, steps within a wave exchange them by
 // lane shuffles, and the steps across waves (partner distance >= 64 R) go
@@ -685,19 +690,19 @@ __device__ __forceinline__ void query_epilogue(const FwdParams& p, QuerySmemT<kR
 // sequence, whatever order the entries came in. Not inlined: inside the
 // per-query unit, where Q^T and O are live, the unrolled network made the
 // compiler spill scalar registers and use scratch.
-template <int R>
-__device__ __attribute__((noinline)) void sort_list(int32_t* s, int n) {
-  constexpr int N = kThreads * R;
+template <int R, typename T = int32_t, int NT = kThreads>
+__device__ __attribute__((noinline)) void sort_list(T* s, int n) {
+  constexpr int N = NT * R;
   const int tid = threadIdx.x;
-  int v[R];
+  T v[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int i = tid * R + r;
-    v[r] = i < n ? s[i] : INT32_MAX;
+    v[r] = i < n ? s[i] : std::numeric_limits<T>::max();
   }
   // the element of key position i keeps the smaller of the pair when the
   // pair's run ascends and i is its lower position, or descends and i is not
-  auto keep = [](int mine, int other, int i, int k, int j) {
+  auto keep = [](T mine, T other, int i, int k, int j) {
     const bool up = (i & k) == 0, low = (i & j) == 0;
     return up == low ? min(mine, other) : max(mine, other);
   };
@@ -710,7 +715,7 @@ __device__ __attribute__((noinline)) void sort_list(int32_t* s, int n) {
         for (int r = 0; r < R; ++r) {
           if ((r & j) != 0) continue;
           const int i = tid * R + r;
-          const int a = v[r], b = v[r | j];
+          const T a = v[r], b = v[r | j];
           const bool up = (i & k) == 0;
           v[r] = up ? min(a, b) : max(a, b);
           v[r | j] = up ? max(a, b) : min(a, b);
@@ -718,7 +723,7 @@ __device__ __attribute__((noinline)) void sort_list(int32_t* s, int n) {
       } else if (j < 64 * R) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-          const int o = __shfl_xor(v[r], j / R);
+          const T o = T(__shfl_xor(int(v[r]), j / R));
           v[r] = keep(v[r], o, tid * R + r, k, j);
         }
       } else {
@@ -1116,10 +1121,10 @@ __device__ __forceinline__ void query_stream(const FwdParams& p, int64_t bi, int
 // index kernel 64x1024-1024-128 36.7 -> 13.2 us, 16x4096-4096-128 40.0 ->
 // 21.3, 64x1024-1280-384 101 -> 73 (A/B, same box).
 // The one-wave kernel's list holds this many slots per query (queries with
-// topk up to it run one wave each). Against the 4-wave per-query kernel:
-// topk 128 1365 -> 1102 us/call at 64 x 1024 queries, topk 640 1232 -> 1260
-// at 1 x 16384 (a longer list amortises that kernel's start), so the cap sits
-// between them.
+// topk up to it run one wave each): what eight work-groups per CU leave of
+// LDS is 832. Longer unsplit queries run in sa_fwd_waves_kernel over long
+// caches, and where tiles can be shared in the 4-wave kernel, whose launch also
+// makes the tile order.
 constexpr int kWaveMaxTopk = 384;
 constexpr int kIdxThreadsNarrow = 512;
 constexpr int kIdxVecNarrow = 4;    // index vectors per thread per round
@@ -2015,6 +2020,300 @@ __global__ void __launch_bounds__(64, 2) sa_fwd_wave_kernel(const FwdParams p) {
     }
   }
   wave_epilogue(p, sm.tile, bi, mi, m_run, l_run, oacc);
+}
+
+// ============================================================================
+// per-query launch over long caches: W waves per query
+// ============================================================================
+// Unsplit queries of 385 to 2 048 slots whose kv is too long for shared tiles
+// (kv_len > kMaxTileKv, so at least 16 MiB per batch). One work-group of W
+// waves per query; wave w runs every W-th 16-row step of the query's sorted
+// rows as the wave kernel does, in a buffer of its own and with no barrier, and
+// the waves merge their states at the end.
+// Bound: the gathers beyond L2 (7.7 TB/s from the Infinity Cache), so what
+// counts is how many of them hit: the resident queries sweep their batch's
+// rows in ascending order together, and a row that two queries of an XCD name
+// at about the same time is fetched once. With 16 KiB of buffer per wave and
+// an 8 KiB list, eight waves share a CU, so 1 024 queries (W = 2) or 2 048 (W =
+// 1) are resident at once, against 512 of the four-wave kernel, and two waves
+// per SIMD hide each other's gathers. Measured against that kernel: 16 381
+// queries over 20 480 rows, topk 640 1 172 -> 829 us; 16 x 512 over 20 000, 500
+// 496 -> 380; 300 over 131 072, 2 000 148 -> 97; 1 021 over 131 072, 2 048 258 ->
+// 246 (there a row's two namers on an XCD are some 2 000 rows apart in their
+// sweeps, about what an L2 holds).
+// LDS rows are 1 KiB without padding (W = 2 fills 40 KiB exactly); row r's
+// 16-byte chunk c sits at c ^ f(r), f(r) = 2 (r & 7) | r >> 3: the 16 rows of a
+// K fragment read differ in all four bits and the 8 rows of a transposing V
+// read in the upper three, so both hit every bank once. Each row's gather
+// loads, per lane, the chunk that belongs at its position.
+template <int W>
+struct WavesSmem {
+  static constexpr int kCap = W == 1 ? 1024 : 2048;  // slots
+  uint8_t tile[W][kWRows * kRowBytes];
+  uint32_t list[kCap];
+};
+static_assert(8 * sizeof(WavesSmem<1>) <= 160 * 1024 && 4 * sizeof(WavesSmem<2>) <= 160 * 1024 &&
+                  2 * sizeof(WavesSmem<4>) <= 160 * 1024,
+              "eight waves per CU");
+constexpr int kWavesMaxTopk = 2048;
+
+template <int W>
+__global__ void __launch_bounds__(64 * W, 2) sa_fwd_waves_kernel(const FwdParams p) {
+  using Smem = WavesSmem<W>;
+  __shared__ __attribute__((aligned(1024))) Smem sm;
+  constexpr int kT = 64 * W;
+  constexpr int kSlots = Smem::kCap / kT;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15;
+  const int g = lane >> 4;
+  const int64_t bi = blockIdx.x / p.m;
+  const int64_t mi = blockIdx.x - bi * p.m;
+  const int topk = int(p.topk);
+  const uint32_t row_bytes = uint32_t(p.skv_n * 2);
+
+  // ---- indices, then Q^T (as in the wave kernel) -----------------------------------------
+  const int32_t* irow = p.idx + bi * p.si_b + mi * p.si_m;
+  int raw[kSlots];
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) raw[i] = kT * i + tid < topk ? irow[kT * i + tid] : -1;
+  bf16x8 qf[kDim / 32];
+  const __bf16* qrow = p.q + bi * p.sq_b + mi * p.sq_m + int64_t(n) * p.sq_h + 8 * g;
+#pragma unroll
+  for (int s = 0; s < kDim / 32; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s);
+
+  // ---- compaction (in any order) and sort; the count in a tile row, free so far -----------
+  int* const s_cnt = reinterpret_cast<int*>(sm.tile[0]);
+  if (tid == 0) *s_cnt = 0;
+  lds_barrier();
+  {
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int mine = 0;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) {
+      const int v = raw[i];
+      const bool ok = (v >= 0) && (int64_t(v) < p.kv_len);
+      bad |= (!ok && v != -1);
+      mine += __popcll(__ballot(ok));
+    }
+    if (bad && p.err != nullptr) flag_bad_index(p.err);
+    int pos = 0;
+    if (lane == 0) pos = atomicAdd(s_cnt, mine);
+    pos = __builtin_amdgcn_readfirstlane(pos);
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) {
+      const int v = raw[i];
+      const bool ok = (v >= 0) && (int64_t(v) < p.kv_len);
+      const unsigned long long bm = __ballot(ok);
+      if (ok) sm.list[pos + __popcll(bm & below)] = uint32_t(v) * row_bytes;
+      pos += __popcll(bm);
+    }
+  }
+  lds_barrier();
+  const int cnt = __builtin_amdgcn_readfirstlane(*s_cnt);
+  if constexpr (W == 1) {
+    if (cnt <= 512)
+      sort_list_wave<8>(sm.list, cnt);
+    else
+      sort_list_wave<16>(sm.list, cnt);
+  } else {
+    if (4 * cnt <= Smem::kCap)
+      sort_list<kSlots / 4, uint32_t, kT>(sm.list, cnt);
+    else if (2 * cnt <= Smem::kCap)
+      sort_list<kSlots / 2, uint32_t, kT>(sm.list, cnt);
+    else
+      sort_list<kSlots, uint32_t, kT>(sm.list, cnt);
+  }
+  const int ns = (cnt + kWRows - 1) / kWRows;
+
+  // ---- steps wave, wave + W, ... -----------------------------------------------------------
+  uint8_t* const tile = sm.tile[wave];
+  const uint32_t lds_rows =
+      __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>((lds_u8_t*)tile)));
+  const uint8_t* kvb = reinterpret_cast<const uint8_t*>(p.kv + bi * p.skv_b);
+  // Lane l < 16 holds the entry of step s's row l; entries past the last valid
+  // one take the first entry's row, whose scores are masked.
+  auto step_rows = [&](int s) {
+    const int e = s * kWRows + n;
+    return sm.list[e < cnt ? e : 0];
+  };
+  auto f_of = [](int r) { return 2 * (r & 7) | r >> 3; };
+  auto gather = [&](uint32_t rv) {
+#pragma unroll
+    for (int i = 0; i < kWRows; ++i) {
+      const uint32_t off = uint32_t(__builtin_amdgcn_readlane(int(rv), i));
+      lds_dma_row(kvb + off, 16 * (lane ^ f_of(i)), lds_rows + uint32_t(i * kRowBytes));
+    }
+  };
+  f32x4 oacc[32];
+  float m_run = -INFINITY, l_run = 0.f;
+#pragma unroll
+  for (int blk = 0; blk < 32; ++blk) oacc[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // K: row n, chunk (4k + g) ^ f(n); V: row 4g + n / 4, chunk (2 blk + (n & 3) / 2) ^ f
+  const uint32_t kbase = uint32_t(n * kRowBytes + 16 * (g ^ f_of(n)));
+  const int vr = 4 * g + (n >> 2);
+  const uint32_t vbase = uint32_t(vr * kRowBytes + 16 * (((n >> 1) & 1) ^ f_of(vr)) + 8 * (n & 1));
+  auto k_at = [&](int k) { return tile + ((kbase ^ uint32_t(64 * (k & 3))) + 256 * (k >> 2)); };
+  auto v_at = [&](int b) { return tile + ((vbase ^ uint32_t(32 * (b & 7))) + 256 * (b >> 3)); };
+  if (wave < ns) gather(step_rows(wave));
+  for (int s = wave; s < ns; s += W) {
+    const uint32_t rv = s + W < ns ? step_rows(s + W) : 0u;
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this step's rows have landed
+    asm volatile("" ::: "memory");
+    const int nrows = cnt - s * kWRows;
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    bf16x8 kf[4];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) kf[k] = *reinterpret_cast<const bf16x8*>(k_at(k));
+#pragma unroll
+    for (int k = 0; k < kDim / 32; ++k) {
+      if (k + 3 < kDim / 32) kf[(k + 3) & 3] = *reinterpret_cast<const bf16x8*>(k_at(k + 3));
+      if (k & 1)
+        sb = mfma_16x16x32(kf[k & 3], qf[k], sb);
+      else
+        sa = mfma_16x16x32(kf[k & 3], qf[k], sa);
+      __builtin_amdgcn_sched_barrier(0);  // keep the interleave
+    }
+    bf16x4 vf[kWVAhead];
+#pragma unroll
+    for (int i = 0; i < kWVAhead; ++i) vf[i] = lds_read_tr16(v_at(i));
+
+    // online softmax, as in the wave kernel
+    float sv[4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      sv[k] = (4 * g + k < nrows) ? (sa[k] + sb[k]) * p.scale_log2 : -INFINITY;
+      mx = fmaxf(mx, sv[k]);
+    }
+    mx = wave_max16(mx);  // finite: the step's row 0 is valid
+    float alpha = 1.f;
+    if (mx > m_run + kRescaleLog2) {
+      alpha = m_run == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mx);
+      m_run = mx;
+    }
+    float psum = 0.f;
+    bf16x4 pb;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float pk = __builtin_amdgcn_exp2f(sv[k] - m_run);
+      psum += pk;
+      pb[k] = static_cast<__bf16>(pk);
+    }
+    l_run = l_run * alpha + psum;
+    if (__any(alpha != 1.f)) {
+      float ak[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ak[k] = __shfl(alpha, 4 * g + k);
+#pragma unroll
+      for (int blk = 0; blk < 32; ++blk)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) oacc[blk][k] *= ak[k];
+    }
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const bf16x4 v = vf[i % kWVAhead];
+      if (i + kWVAhead < 32) vf[i % kWVAhead] = lds_read_tr16(v_at(i + kWVAhead));
+      oacc[i] = mfma_16x16x16(pb, v, oacc[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (s + W < ns) {  // every read of the buffer is complete
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      gather(rv);
+    }
+  }
+
+  // ---- merge the waves' states -----------------------------------------------------------------
+  // (m, l) of each wave and head through the list, free by now
+  float m_all = m_run, l_all = wave_sum16(l_run);
+  if constexpr (W > 1) {
+    float2* const s_ml = reinterpret_cast<float2*>(sm.list);
+    lds_barrier();  // every wave is past its last read of the list
+    if (g == 0) s_ml[wave * kHeads + n] = make_float2(m_run, l_all);
+    lds_barrier();
+    float2 ml[W];
+    m_all = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      ml[w] = s_ml[w * kHeads + n];
+      m_all = fmaxf(m_all, ml[w].x);
+    }
+    l_all = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w)  // a wave without a step: m = -inf, l = 0
+      l_all += ml[w].x == -INFINITY ? 0.f : ml[w].y * __builtin_amdgcn_exp2f(ml[w].x - m_all);
+  }
+  float lse;
+  float f = sink_fold(m_all, l_all, p.sink[n] * kLog2e, lse);
+  if (p.lse != nullptr && tid < 16)
+    p.lse[bi * p.sl_b + mi * p.sl_m + int64_t(n) * p.sl_h] = lse;
+  if (W > 1) f = m_run == -INFINITY ? 0.f : f * __builtin_amdgcn_exp2f(m_run - m_all);
+  float fj[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) fj[j] = __shfl(f, 4 * g + j);
+#pragma unroll
+  for (int blk = 0; blk < 32; ++blk)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) oacc[blk][j] *= fj[j];
+  // Sum over the waves, each keeping 32 / W column blocks: with partner wave ^
+  // bit, the half of the blocks that the partner keeps goes through this
+  // wave's buffer.
+  int col0 = 0;  // first column of the kept blocks
+  uint8_t* stage = tile;
+  auto exchange = [&](auto kept, int bit) {
+    constexpr int kN = decltype(kept)::value;
+    const bool upper = (wave & bit) != 0;
+    f32x4* const own = reinterpret_cast<f32x4*>(tile);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) own[i * 64 + lane] = upper ? oacc[i] : oacc[kN + i];
+    lds_barrier();
+    stage = sm.tile[wave ^ bit];
+    const f32x4* const other = reinterpret_cast<const f32x4*>(stage);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) oacc[i] = (upper ? oacc[kN + i] : oacc[i]) + other[i * 64 + lane];
+    col0 += upper ? 16 * kN : 0;
+  };
+  if constexpr (W >= 2) exchange(std::integral_constant<int, 16>{}, 1);
+  if constexpr (W >= 4) {
+    lds_barrier();  // the partner is done with this wave's buffer
+    exchange(std::integral_constant<int, 8>{}, 2);
+  }
+  // Output by whole (part) rows through LDS, as in the wave kernel, in the
+  // buffer that only this wave has just read (W = 1: its own and the list)
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int kBlks = 32 / W;
+  constexpr int kPitch = 32 * kBlks + (W == 1 ? 48 : 16);  // 16 heads: every bank once
+  static_assert(kHeads * kPitch <= (W == 1 ? int(sizeof(Smem)) : kWRows * kRowBytes), "rows fit");
+  const bool odd = (n & 1) != 0;
+  uint8_t* const r0 = stage + (4 * g + (odd ? 2 : 0)) * kPitch + 2 * (n & ~1);
+  auto swap = [](float x) {  // the value of lane n ^ 1
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
+  };
+#pragma unroll
+  for (int blk = 0; blk < kBlks; ++blk) {
+    const float x0 = swap(odd ? oacc[blk][0] : oacc[blk][2]);
+    const float x1 = swap(odd ? oacc[blk][1] : oacc[blk][3]);
+    const f32x2 a = odd ? f32x2{x0, oacc[blk][2]} : f32x2{oacc[blk][0], x0};
+    const f32x2 b = odd ? f32x2{x1, oacc[blk][3]} : f32x2{oacc[blk][1], x1};
+    *reinterpret_cast<bf16x2*>(r0 + 32 * blk) = __builtin_convertvector(a, bf16x2);
+    *reinterpret_cast<bf16x2*>(r0 + kPitch + 32 * blk) = __builtin_convertvector(b, bf16x2);
+  }
+  asm volatile("" ::: "memory");  // one wave: its LDS operations run in order
+  constexpr int kLanes = 2 * kBlks;          // 16-byte lanes per head's part row
+  constexpr int kPer = 64 / kLanes;          // heads per store
+  __bf16* const orow = p.o + bi * p.so_b + mi * p.so_m + col0 + 8 * (lane % kLanes);
+#pragma unroll
+  for (int i = 0; i < kHeads / kPer; ++i) {
+    const int h = i * kPer + lane / kLanes;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + h * kPitch + 16 * (lane % kLanes));
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(orow + int64_t(h) * p.so_h));
+  }
 }
 
 // ============================================================================
@@ -3048,6 +3347,11 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
       what == Launch::kCall && plan.nsplit == 1 && a->topk <= kWaveMaxTopk && a->kv_len > 0 &&
       (a->kv_len - 1) * a->skv[1] * 2 + 2 * kDim <= int64_t(UINT32_MAX);
 
+  const bool waves_ok =
+      what == Launch::kCall && plan.nsplit == 1 && a->topk > kWaveMaxTopk &&
+      a->topk <= kWavesMaxTopk && a->kv_len > sa::kMaxTileKv &&
+      (a->kv_len - 1) * a->skv[1] * 2 + 2 * kDim <= int64_t(UINT32_MAX);
+
   // The per-query kernel; two work-groups per CU once there are at least two
   // per CU to run.
   auto launch_query = [&]() -> int {
@@ -3055,6 +3359,20 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
       return run(SA_KERNEL_WAVE, fn(sa_fwd_wave_kernel),
                  dim3(unsigned(p.nblocks)), dim3(64), 0, &p);
     const dim3 grid(unsigned(p.nblocks)), block(kThreads);
+    // Long caches (never shared tiles, whatever the flags): as many waves per
+    // query as keep the SIMDs busy. W = 1 / 2 / 4 (four-wave kernel), us per
+    // call: 16 381 queries, topk 640 [825] / 1 100 / 1 107 (1 168); 1 600,
+    // 700 [133] / 139 / 147 (153); 1 021, 2 048 [247] / 263 for 2 / 4 (256);
+    // 512, 1 000 [64] / 71 (68); 300, 2 000 106 / [99] (150).
+    if (p.meta == nullptr && waves_ok) {
+      const int w = a->topk <= WavesSmem<1>::kCap && p.nblocks >= 6 * int64_t(cus) ? 1
+                    : p.nblocks >= 2 * int64_t(cus)                               ? 2
+                                                                                  : 4;
+      const void* k = w == 1   ? fn(sa_fwd_waves_kernel<1>)
+                      : w == 2 ? fn(sa_fwd_waves_kernel<2>)
+                               : fn(sa_fwd_waves_kernel<4>);
+      return run(SA_KERNEL_QUERY, k, grid, dim3(unsigned(64 * w)), 0, &p);
+    }
     const bool two = p.nblocks >= 2 * int64_t(cus);
     const void* k = p.meta != nullptr
                         ? (two ? fn(sa_fwd_query_kernel<2, true>) : fn(sa_fwd_query_kernel<4, true>))

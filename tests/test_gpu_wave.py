@@ -245,3 +245,38 @@ def test_index_bitmap_mode_bad_index(gpu_sa):
     ok[0, 3, 10] = -1
     ok[0, 9, 20] = -1
     check(o, sparse_attn_fp64(q, kv, sink, ok, sc), "bitmap mode, bad index")
+
+
+@pytest.mark.parametrize("b,m,kv_len,topk,minus1", [
+    (1, 261, 16385, 385, 0.1),    # four waves per query; the shortest list and cache
+    (2, 200, 20000, 2048, 0.0),   # four waves, the longest list
+    (1, 800, 40000, 1025, 0.3),   # two waves, a list past one wave's capacity
+    (3, 256, 17000, 2000, 0.9),   # two waves, lists that need fewer keys in the sort
+    (1, 1537, 16400, 1024, 0.05), # one wave per query, its longest list
+    (1, 1600, 30000, 390, 0.0),   # one wave, the short sort
+])
+def test_long_cache_waves(gpu_sa, b, m, kv_len, topk, minus1):
+    """Unsplit queries of 385 to 2 048 slots over caches too long for shared
+    tiles: W waves per query (by the number of queries), empty queries, single
+    rows, a step's worth, duplicates; sampled queries, o and lse, against the
+    float64 oracle, and the same bits from a second run."""
+    q, kv, sink, idx, sc = case(b, m, kv_len, topk, seed=topk + m, minus1=minus1)
+    idx[0, 0] = -1                     # nothing valid: every wave without a step
+    idx[0, 1] = -1
+    idx[0, 1, 7] = kv_len - 1          # one row: one wave with a step
+    idx[0, 2, 17:] = -1                # two steps
+    idx[0, 3] = 5                      # one row, topk times
+    idx[-1, m - 1, ::2] = -1
+    if expect_plan(q, kv, idx, 0, tiles=False)["nsplit"] != 1:
+        pytest.skip("split on this device")
+    o, lse, mask, err, _ = run(q, kv, sink, idx, sc, with_lse=True)
+    assert err == 0 and mask == QUERY
+    sel = [0, 1, 2, 3, 4, m // 2, m - 2, m - 1]
+    o_ref, lse_ref = sparse_attn_lse_fp64(q[:, sel], kv, sink, idx[:, sel], sc)
+    check(o.cpu()[:, sel], o_ref, f"waves topk {topk}")
+    assert torch.all(o.cpu()[0, 0] == 0)
+    assert np.abs(lse.double().cpu().numpy()[:, sel] - lse_ref).max() <= 2e-3
+    o2, lse2, _, _, _ = run(q, kv, sink, idx, sc, with_lse=True)
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+    idx[0, 4, 3] = kv_len
+    assert run(q, kv, sink, idx, sc)[3] == 1
