@@ -590,8 +590,7 @@ def moe_gemm_kernel(M, N, E, topk, gated):
     avg = P / E
     g = "true" if gated else "false"
     one_round = min(E, P) * math.ceil((avg + 1.5 * math.sqrt(avg)) / 256) * (N // 32) <= 256
-    if avg > 24.0 or (one_round and avg >= 4.0) or (N <= 512 and avg > 6.0) or \
-            (N % 256 != 0 and avg > 8.0):
+    if avg > 24.0 or (avg > 12.0 and (one_round or N <= 512)) or (N % 256 != 0 and avg > 8.0):
         return f"fm_gemm_kernel<{g}>"
     pb = 2 if avg > 12.0 else 1
     if N % 256 == 0:

@@ -98,14 +98,15 @@ inline size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 //   Short last tiles narrow against wide: M = 4096, E = 8 [134] / 175; M =
 //   1500, K = 2048, N = 1408, E = 16, topk = 4 169 / [164]; M = 4001, E = 64,
 //   topk = 6 481 / [385].
-// The streamed tiles read each weight once into one short-lived work-group and
-// win where the weights of many experts are the traffic (E = 64, M = 64: 163
-// against 183; M = 8: 108 against 122) and below 4 pairs per expert; with at
-// most one narrow item per CU fm_gemm_kernel wins from there (E = 8, M = 16: 35
-// against 38; M = 64: 36 against 41), and from 6 or 8 pairs where the streamed
-// kernel's own pipelines are short or absent (N <= 512: E = 128, M = 100, topk
-// = 8 93 against 107; N not a multiple of 256: E = 16, M = 60, topk = 4,
-// N = 1408 79 against 90).
+// The streamed tiles win where the weights of many experts are the traffic
+// (E = 64, topk = 6: M = 64 152 against 183, M = 8 94 against 122) and up to 12
+// pairs per expert in general (E = 8, topk = 2, M = 16 29 against 30; K = 4096,
+// N = 512, E = 32, topk = 4, M = 60 88 against 102). Past that they need two
+// pair blocks per tile, and fm_gemm_kernel wins with at most one narrow item
+// per CU (E = 8, topk = 2, M = 64 34 against 41) or short K loops in the down
+// GEMM (N <= 512: E = 128, topk = 8, M = 200 97 against 117), and from 8
+// pairs where N is not a multiple of 256 (E = 16, topk = 4, N = 1408, M = 60 79
+// against 90).
 void choose_tiles(const fm_args* a, Plan& p) {
   const double n = double(p.P) / double(a->E), sd = sqrt(n);
   auto tiles = [&](double pairs, int rows) { return double(p.nonempty) * ceil(pairs / rows); };
@@ -118,7 +119,7 @@ void choose_tiles(const fm_args* a, Plan& p) {
   else if (a->flags & FM_FLAG_SMALL_TILES)
     p.gemm = false;
   else
-    p.gemm = n > 24.0 || (one_round && n >= 4.0) || (a->N <= 512 && n > 6.0) ||
+    p.gemm = n > 24.0 || (n > 12.0 && (one_round || a->N <= 512)) ||
              (a->N % 256 != 0 && n > 8.0);
   // 16 or 32 pairs per small tile (64 only when forced)
   p.pb = n > 24.0 && a->N % 256 == 0 ? 4 : n > 12.0 ? 2 : 1;
@@ -1166,7 +1167,7 @@ __global__ void __launch_bounds__(256) fm_skinny_kernel(const GemmParams p) {
 // but every operand reaches the MFMAs through LDS, filled by LDS-DMA in
 // stages of 256 k: one instruction moves two rows' 512 contiguous bytes, so
 // each weight row streams from HBM in long runs. Stages go through a ring of
-// 3-6 buffers (all but one in flight); all waits are explicit (no
+// 3 or 4 buffers (all but one in flight); all waits are explicit (no
 // compiler-tracked load shares the vmcnt counter with the DMAs). Pair rows
 // past the tile's last pair are not loaded. Row r's 16-byte chunk c sits
 // at position c ^ (r & 15) of its 512-byte line, so the 16 rows of a 16x16x32
@@ -1182,8 +1183,11 @@ __global__ void __launch_bounds__(256, 1) fm_stream_kernel(const GemmParams p) {
   constexpr int kBuf = (kRowsW + kRowsP) * kStLine; // one stage
   constexpr int kDmaW = kRowsW / 2 / 4;             // weight DMAs per wave per stage (4)
   constexpr int kDmaP = kRowsP / 2 / 4;             // pair DMAs per wave per stage (2 PB)
-  // ring depth: as many stages as 144 KiB of LDS hold (6, 4, 3)
-  constexpr int kStBufs = (144 * 1024) / kBuf;
+  // ring depth: two work-groups per CU with three stages of one pair block
+  // each, whose starts and partial-sum barriers overlap the other's loads (one
+  // with six before: M = 64, E = 64, topk = 6 161 -> 151 us per call, M = 4
+  // 69 -> 60); else one with four or three
+  constexpr int kStBufs = PB == 1 ? 3 : (144 * 1024) / kBuf;
   static_assert(kStBufs >= 3 && 4 * 2 * PB * 64 * 16 <= kBuf, "ring and reduction fit");
   __shared__ __attribute__((aligned(1024))) uint8_t s_buf[kStBufs * kBuf];
   const int tid = threadIdx.x;
@@ -1507,13 +1511,27 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   }
   g1.ct_per_wg = g2.ct_per_wg = 1;
   if (streamed) {
-    // a streaming work-group runs several column tiles in one pipeline, so its
-    // start (tile table -> pair list -> first DMA) is paid once per
-    // several: about 1024 work-groups per launch, whole column tiles each
+    // A streaming work-group runs several column tiles in one pipeline, so its
+    // start (tile table -> pair list -> first DMA), about four stages' time,
+    // is paid once per several: as many as make the rounds of work-groups (half
+    // a round more for their spread) times a work-group's time least, for the
+    // expected number of tiles. E = 64, topk = 6, us per call, 1 / 2 / 4 / 8
+    // gate-up column tiles: M = 64 162 / 152 / 151 / 155, M = 128 171 / 158 /
+    // 168 / -.
+    const double used = double(a->E) * (1.0 - pow(1.0 - double(a->topk) / double(a->E), double(a->M)));
+    const double mean = double(pl.P) / used;
+    const double est = used * (1.0 + 0.5 * erfc((pl.tile_rows + 0.5 - mean) / sqrt(2.0 * mean)));
+    const double slots = pl.pb == 1 ? 2.0 * kCus : kCus;
     for (GemmParams* g : {&g1, &g2}) {
-      int c = 1;
-      while (c * 2 <= g->col_tiles && pl.max_tiles * (g->col_tiles / (c * 2)) >= 1024) c *= 2;
-      g->ct_per_wg = c;
+      double best = 0.0;
+      for (int c = 1; c <= g->col_tiles; c *= 2) {
+        const double wgs = est * ((g->col_tiles + c - 1) / c);
+        const double t = (ceil(wgs / slots) + 0.5) * (4 + c * (g->kin / kStK));
+        if (c == 1 || t < best) {
+          best = t;
+          g->ct_per_wg = c;
+        }
+      }
     }
   }
   auto grid_of = [&](const GemmParams& g) {
