@@ -307,6 +307,15 @@ def cpu_baseline(cpu_inputs, target_s=4.0, runs=3):
             "us_per_call_extrapolated": round(dt / nq * b * m * 1e6, 1)}
 
 
+def kernel_names(name):
+    """KERNEL_NAMES for a workload: the per-query launch of unsplit queries of
+    385 to 2 048 slots over more than 16 384 rows is sa_fwd_waves_kernel."""
+    cfg = wl.CONFIGS.get(name)
+    if cfg and cfg.kv_len > 16384 and 384 < cfg.topk <= 2048 and cfg.b * cfg.m >= 256:
+        return dict(KERNEL_NAMES, query="sa_fwd_waves_kernel")
+    return KERNEL_NAMES
+
+
 def roofline(name, flops, compulsory, times, shares, us_per_call):
     """The dominant kernel's algorithmic rate: its share of the call's flops
     (or compulsory bytes) over its average launch duration, measured in this
@@ -333,7 +342,8 @@ def roofline(name, flops, compulsory, times, shares, us_per_call):
         roof["traffic_note"] = ("no traffic profile for this workload" if not tr else
                                 f"profiles/traffic.json was measured on sources {tr.get('sources')}, "
                                 f"this build is {digest}")
-    roof["kernel"] = KERNEL_NAMES[dom]
+    names = kernel_names(name)
+    roof["kernel"] = names[dom]
     roof["kernel_us"] = round(times[dom] * 1e3, 2)
     roof["kernel_timing"] = "HIP events taking the dispatch timestamps (hipExtLaunchKernel)"
     over = times[dom] * 1e3 / us_per_call
@@ -348,10 +358,10 @@ def roofline(name, flops, compulsory, times, shares, us_per_call):
                              f"us_per_call {us_per_call} (separate loops; within "
                              f"{100 * KERNEL_OVER_CALL_TOL:.0f} %)")
     roof["work_share"] = round(share, 4)
-    roof["kernel_us_all"] = {KERNEL_NAMES[k]: round(v * 1e3, 2) for k, v in times.items()}
+    roof["kernel_us_all"] = {names[k]: round(v * 1e3, 2) for k, v in times.items()}
     roof["sources"] = digest
     prof = _profile_rec(KERNEL_TRACE_JSON, name)
-    if prof and prof.get("kernel", "").split("<")[0] == KERNEL_NAMES[dom]:
+    if prof and prof.get("kernel", "").split("<")[0] == names[dom]:
         roof["profile"] = {"trace": prof.get("profile"), "kernel": prof.get("kernel"),
                            "kernel_us": prof["avg_us"], "dispatches": prof.get("calls"),
                            "frac": round(work / (prof["avg_us"] * 1e-6) / peak, 4),

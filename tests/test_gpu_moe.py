@@ -191,6 +191,18 @@ def test_routing_over_work_groups(gpu_sa, shape):
           f"{shape}")
 
 
+def test_gemm_silu_over_its_range(gpu_sa):
+    """Gate values over about +-100: both tails of silu, where the exponential
+    overflows or vanishes, against the oracle's exact one."""
+    M, K, N, E, topk = 300, 512, 256, 4, 2
+    hidden, w1, w2, score = make_inputs(M, K, N, E, seed=15)
+    w1, w2 = w1 * 56, w2 * 1e-3
+    gate = hidden.float() @ w1[0, :N].float().t()
+    assert gate.min() < -90 and gate.max() > 90
+    out = op(hidden, w1, w2, score, topk)
+    check(out, fused_moe_ref(*cpu(hidden, w1, w2, score), topk), "wide gate range")
+
+
 @pytest.mark.parametrize("M", [16, 64])
 def test_streamed_final_sum_forms(gpu_sa, M):
     """Streamed tiles where fm_gemm_kernel is the default: the atomic and the
