@@ -203,6 +203,33 @@ def test_gemm_silu_over_its_range(gpu_sa):
     check(out, fused_moe_ref(*cpu(hidden, w1, w2, score), topk), "wide gate range")
 
 
+@pytest.mark.parametrize("flags", [0, 1, 4], ids=["narrow", "large", "big"])
+def test_gemm_silu_of_every_bf16_gate(gpu_sa, flags):
+    """Token t of expert 0 has gate value w1[j, t] at feature j, up value 1 and
+    w2 = 1, so the output is silu of all finite bf16 values: fm_gemm_kernel's
+    has the bits of the streamed kernel's, and lies within half a bf16 step
+    (2^-8 of the value at most) and 4 float32 ulp of float64's wherever 1 +
+    exp(-x) and the result are normal float32 numbers (below -88.7 the
+    exponential overflows: 0)."""
+    n = 256
+    x = torch.arange(n * n, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(n, n)
+    x = torch.where(x.isfinite(), x, torch.zeros_like(x))
+    w1 = torch.cat([x, torch.ones_like(x)])[None].to(DEV)
+    eye = torch.eye(n, dtype=torch.bfloat16, device=DEV)
+    score = torch.zeros(n, 1, dtype=torch.bfloat16, device=DEV)
+    got = op(eye, w1, eye[None].contiguous(), score, 1, flags=flags)
+    streamed = op(eye, w1, eye[None].contiguous(), score, 1, flags=2 | 8)
+    bad = torch.nonzero(got.t().cpu().view(torch.int16) != streamed.t().cpu().view(torch.int16))
+    say("  differing gates:", [(x[i, j].item(), got[j, i].item(), streamed[j, i].item())
+                               for i, j in bad.tolist()[:8]])
+    assert len(bad) == 0
+    xd, y = x.double(), got.t().cpu().double()
+    exact = xd / (1 + torch.exp(-xd))
+    normal = (xd > -88.7) & (xd.abs() > 2.0 ** -120)
+    assert ((y - exact).abs() <= (2 ** -8 + 2 ** -21) * exact.abs())[normal].all()
+    assert (y[xd < -88.7].abs() <= 1e-36).all()
+
+
 @pytest.mark.parametrize("M", [16, 64])
 def test_streamed_final_sum_forms(gpu_sa, M):
     """Streamed tiles where fm_gemm_kernel is the default: the atomic and the
