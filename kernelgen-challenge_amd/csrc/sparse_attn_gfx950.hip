@@ -2243,8 +2243,9 @@ __global__ void __launch_bounds__(64 * W, 2) sa_fwd_waves_kernel(const FwdParams
     }
     l_all = 0.f;
 #pragma unroll
-    for (int w = 0; w < W; ++w)  // a wave without a step: m = -inf, l = 0
-      l_all += ml[w].x == -INFINITY ? 0.f : ml[w].y * __builtin_amdgcn_exp2f(ml[w].x - m_all);
+    for (int w = 0; w < W; ++w)  // m = -inf: l = 0 (no step) or NaN
+      l_all += ml[w].x == -INFINITY ? ml[w].y
+                                    : ml[w].y * __builtin_amdgcn_exp2f(ml[w].x - m_all);
   }
   float lse;
   float f = sink_fold(m_all, l_all, p.sink[n] * kLog2e, lse);

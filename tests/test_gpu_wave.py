@@ -280,3 +280,33 @@ def test_long_cache_waves(gpu_sa, b, m, kv_len, topk, minus1):
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
     idx[0, 4, 3] = kv_len
     assert run(q, kv, sink, idx, sc)[3] == 1
+
+
+# W = 4, 2 and 1 waves per query
+LONG_CACHE = [(300, 2000), (520, 1000), (1540, 400)]
+
+
+@pytest.mark.parametrize("m,topk", LONG_CACHE)
+def test_long_cache_waves_keep_nan(gpu_sa, m, topk):
+    """A wave whose scores are all NaN has no maximum, but its NaN reaches the
+    query's lse as well as its o, whatever the other waves hold; other heads
+    and queries are untouched."""
+    q, kv, sink, idx, sc = case(1, m, 16400, topk, seed=topk, minus1=0.1)
+    idx[0, 1] = -1
+    idx[0, 1, 7] = 16399             # one row, which is NaN
+    idx[0, 4] = -1
+    idx[0, 4, :32] = torch.arange(32, dtype=torch.int32)
+    idx[0, 4, 16:32] = 16399         # the second of two steps is that row
+    idx[0, 5:][idx[0, 5:] == 16399] = 3
+    q[0, 2, 3] = float("nan")        # one head's scores
+    idx[0, :1][idx[0, :1] == 16399] = 3
+    idx[0, 2:4][idx[0, 2:4] == 16399] = 3
+    kv[0, 16399, 5] = float("nan")
+    if expect_plan(q, kv, idx, 0, tiles=False)["nsplit"] != 1:
+        pytest.skip("split on this device")
+    o, lse, mask, err, _ = run(q, kv, sink, idx, sc, with_lse=True)
+    assert err == 0 and mask == QUERY
+    nan = torch.zeros(m, 16, dtype=torch.bool)
+    nan[1] = nan[4] = nan[2, 3] = True
+    assert torch.equal(lse[0].isnan().cpu(), nan)
+    assert torch.equal(o[0].isnan().cpu(), nan[..., None].expand(m, 16, 512))
