@@ -1975,18 +1975,20 @@ __global__ void __launch_bounds__(64, 2) sa_fwd_wave_kernel(const FwdParams p) {
       sv[k] = (4 * g + k < nrows) ? (sa[k] + sb[k]) * p.scale_log2 : -INFINITY;
       mx = fmaxf(mx, sv[k]);
     }
-    mx = wave_max16(mx);  // finite: the step's row 0 is valid
+    mx = wave_max16(mx);
     float alpha = 1.f;
     if (mx > m_run + kRescaleLog2) {
       // (O, l still 0 at first; v_exp_f32 as in the per-query step)
       alpha = m_run == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mx);
       m_run = mx;
     }
+    // No maximum yet: every score so far overflowed to -inf (weight 0) or is NaN.
+    const float mref = m_run == -INFINITY ? 0.f : m_run;
     float psum = 0.f;
     bf16x4 pb;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float pk = __builtin_amdgcn_exp2f(sv[k] - m_run);
+      const float pk = __builtin_amdgcn_exp2f(sv[k] - mref);
       psum += pk;
       pb[k] = static_cast<__bf16>(pk);
     }
@@ -2188,17 +2190,18 @@ __global__ void __launch_bounds__(64 * W, 2) sa_fwd_waves_kernel(const FwdParams
       sv[k] = (4 * g + k < nrows) ? (sa[k] + sb[k]) * p.scale_log2 : -INFINITY;
       mx = fmaxf(mx, sv[k]);
     }
-    mx = wave_max16(mx);  // finite: the step's row 0 is valid
+    mx = wave_max16(mx);
     float alpha = 1.f;
     if (mx > m_run + kRescaleLog2) {
       alpha = m_run == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mx);
       m_run = mx;
     }
+    const float mref = m_run == -INFINITY ? 0.f : m_run;
     float psum = 0.f;
     bf16x4 pb;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float pk = __builtin_amdgcn_exp2f(sv[k] - m_run);
+      const float pk = __builtin_amdgcn_exp2f(sv[k] - mref);
       psum += pk;
       pb[k] = static_cast<__bf16>(pk);
     }
@@ -2243,7 +2246,7 @@ __global__ void __launch_bounds__(64 * W, 2) sa_fwd_waves_kernel(const FwdParams
     }
     l_all = 0.f;
 #pragma unroll
-    for (int w = 0; w < W; ++w)  // m = -inf: l = 0 (no step) or NaN
+    for (int w = 0; w < W; ++w)  // m = -inf: l = 0, or NaN (NaN scores only)
       l_all += ml[w].x == -INFINITY ? ml[w].y
                                     : ml[w].y * __builtin_amdgcn_exp2f(ml[w].x - m_all);
   }

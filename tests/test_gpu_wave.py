@@ -310,3 +310,32 @@ def test_long_cache_waves_keep_nan(gpu_sa, m, topk):
     nan[1] = nan[4] = nan[2, 3] = True
     assert torch.equal(lse[0].isnan().cpu(), nan)
     assert torch.equal(o[0].isnan().cpu(), nan[..., None].expand(m, 16, 512))
+
+
+@pytest.mark.parametrize("m,topk", LONG_CACHE + [(300, 200)])
+def test_long_cache_rows_whose_scores_overflow(gpu_sa, m, topk):
+    """Rows whose scores overflow to -inf weigh nothing, also where they fill a
+    wave's first step or are all the query has: as without them. (topk 200:
+    the one-wave kernel.)"""
+    q, kv, sink, idx, sc = case(1, m, 16400, topk, seed=topk + 1)
+    kv[..., 0] = 0
+    kv[0, 100:116] = 0
+    kv[0, 100:116, 0] = -1e20        # with q's 1e20 a score of -1e40
+    idx[(idx >= 100) & (idx < 116)] = 3
+    q[0, 1:5, :, 0] = 1e20
+    far, near = torch.arange(100, 116), torch.arange(50, 66)
+    idx[0, 1:5] = -1
+    idx[0, 1, :48] = torch.cat([far, torch.arange(200, 232)])         # the first step
+    idx[0, 2, :48] = torch.cat([near, far, torch.arange(200, 216)])   # the second
+    idx[0, 3, :16] = far                                              # all
+    idx[0, 4, :48] = torch.cat([near, torch.arange(80, 96), far])     # the third
+    ref = idx.clone()
+    ref[(ref >= 100) & (ref < 116)] = -1
+    if expect_plan(q, kv, idx, 0, tiles=False)["nsplit"] != 1:
+        pytest.skip("split on this device")
+    o, lse, mask, err, _ = run(q, kv, sink, idx, sc, with_lse=True)
+    assert err == 0 and mask == (QUERY if topk > 384 else WAVE)
+    sel = [0, 1, 2, 3, 4, m - 1]
+    o_ref, lse_ref = sparse_attn_lse_fp64(q[:, sel], kv, sink, ref[:, sel], sc)
+    check(o.cpu()[:, sel], o_ref, f"overflowing scores, topk {topk}")
+    assert np.abs(lse.double().cpu().numpy()[:, sel] - lse_ref).max() <= 2e-3
