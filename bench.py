@@ -589,12 +589,12 @@ MOE_WORKLOADS = [  # track-03/workloads.py:3-12: label, M, K, N, E, topk
 ]
 MOE_KERNEL_NAMES = {"route": "fm_route_kernel", "plan": "fm_plan_kernel",
                     "reduce": "fm_reduce_kernel"}
-MOE_FUSED_ROUTE_TOKENS = 16  # kFusedTokens in csrc/fused_moe_gfx950.hip
+MOE_FUSED_ROUTE_TOKENS = 16  # kFusedTokens in csrc/fm_plan.h
 
 
 def moe_gemm_kernel(M, N, E, topk, gated):
     """The GEMM kernel fused_moe launches for this shape with flags 0: the
-    choice of choose_tiles in csrc/fused_moe_gfx950.hip, restated for the
+    choice of choose_tiles in csrc/fm_plan.h, restated for the
     report (the profiles' kernel traces name the launched kernel)."""
     P = M * topk
     avg = P / E

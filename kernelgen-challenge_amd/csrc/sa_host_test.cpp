@@ -1,6 +1,7 @@
 // sa_host_test.cpp -- g++-only build of the host-side argument validation and
-// split-topk planning (sa_plan.h), exported for CPU unit tests. Not part of the
-// product ABI; the HIP library compiles the same header.
+// planning (sa_plan.h, fm_plan.h), exported for CPU unit tests. Not part of the
+// product ABI; the HIP libraries compile the same headers.
+#include "fm_plan.h"
 #include "sa_plan.h"
 
 extern "C" {
@@ -50,6 +51,18 @@ int sa_host_plan_full(const sa_args* a, int num_cus, int64_t* out) {
   out[10] = int64_t(p.cnts_off);
   out[11] = int64_t(p.part_off);
   return SA_OK;
+}
+
+// out[0..3] = fm_gemm_kernel or not, tile_rows, narrow_rows, pb
+int fm_host_plan(const fm_args* a, int64_t* out) {
+  const int rc = fm::validate(a);
+  if (rc != FM_OK) return rc;
+  const fm::Plan p = fm::make_plan(a);
+  out[0] = p.gemm ? 1 : 0;
+  out[1] = p.tile_rows;
+  out[2] = p.narrow_rows;
+  out[3] = p.pb;
+  return FM_OK;
 }
 
 }  // extern "C"

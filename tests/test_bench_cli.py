@@ -189,3 +189,33 @@ def test_torch_eager_sinkhorn_is_the_track02_oracle():
     for a, b in zip(got, want):
         assert tuple(a.shape) == b.shape
         assert torch.allclose(a, torch.from_numpy(b), rtol=1e-5, atol=1e-6)
+
+
+def test_kernel_names_follow_the_launch_plans():
+    """bench.py restates which kernel a shape launches; the host-side planners
+    (256 CUs) say the same."""
+    import ctypes
+
+    import sa_capi
+    from sa_testutil import host_lib, moe_plan
+    shapes = [w[1:] for w in bench.MOE_WORKLOADS]
+    shapes += [(M, 2048, N, E, topk) for M in (1, 7, 30, 64, 100, 200, 700, 3000)
+               for N in (512, 1024, 1408) for E, topk in ((8, 2), (16, 4), (64, 6), (128, 8))]
+    for M, K, N, E, topk in shapes:
+        p = moe_plan(M, K, N, E, topk)
+        name = bench.moe_gemm_kernel(M, N, E, topk, True)
+        want = "fm_gemm_kernel<true>" if p["gemm"] else \
+            f"fm_{'stream' if N % 256 == 0 else 'skinny'}_kernel<true, {p['pb']}>"
+        assert name == want, (M, K, N, E, topk)
+    for name, c in wl.CONFIGS.items():
+        a = sa_capi.SaArgs()
+        a.q = a.kv = a.sink = a.idx = a.o = 0x10000
+        a.b, a.m, a.h, a.d, a.kv_len, a.topk = c.b, c.m, 16, 512, c.kv_len, c.topk
+        a.sq[:] = a.so[:] = (c.m * 16 * 512, 16 * 512, 512, 1)
+        a.skv[:] = (c.kv_len * 512, 512, 1)
+        a.sidx[:] = (c.m * c.topk, c.topk, 1)
+        a.scale = wl.SCALE
+        out = (ctypes.c_int64 * 12)()
+        assert host_lib().sa_host_plan_full(ctypes.byref(a), 256, out) == sa_capi.SA_OK
+        waves = out[0] == 1 and not out[2] and 384 < c.topk <= 2048 and c.kv_len > 16384
+        assert (bench.kernel_names(name)["query"] == "sa_fwd_waves_kernel") == waves, name

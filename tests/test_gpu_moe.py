@@ -27,6 +27,7 @@ import torch
 
 import sa_capi
 from oracle.fused_moe_ref import fused_moe_fp64, fused_moe_ref
+from sa_testutil import moe_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -146,10 +147,9 @@ def test_every_token_on_one_expert(gpu_sa):
 @pytest.mark.parametrize("shape", [(1500, 512, 256, 8, 2), (700, 1024, 512, 4, 3),
                                    (2048, 2048, 1024, 8, 2), (700, 1280, 384, 4, 3)])
 def test_big_tiles_equal_large_tiles(gpu_sa, shape):
-    """256-pair tiles (8 waves, 32-wide K stages) and 128-pair tiles (4 waves,
-    64-wide stages) run the same MFMA sequence per output element, so they
-    agree bit for bit, with full and ragged tiles, row blocks past the last
-    pair and pair halves without any."""
+    """256-pair and 128-pair tiles run the same MFMA sequence per output element,
+    so they agree bit for bit, with full and ragged tiles, row blocks past the
+    last pair and wave halves without any."""
     M, K, N, E, topk = shape
     hidden, w1, w2, score = make_inputs(M, K, N, E, seed=9)
     big = op(hidden, w1, w2, score, topk, flags=4)
@@ -157,16 +157,22 @@ def test_big_tiles_equal_large_tiles(gpu_sa, shape):
     assert torch.equal(big, large)
 
 
-@pytest.mark.parametrize("counts,K,N", [
-    ((1, 32, 33, 64), 256, 128), ((65, 128, 129, 0, 255, 256), 256, 128),
-    ((256, 257, 384, 385, 512, 640), 512, 128), ((300,) * 20 + (100,) * 44, 256, 2048),
-    ((17, 200, 256, 31) * 8, 512, 640)])
-def test_gemm_tiles_at_their_edges(gpu_sa, counts, K, N):
+@pytest.mark.parametrize("narrow,counts,K,N", [
+    (256, (1, 32, 33, 64), 256, 128), (256, (65, 128, 129, 0, 255, 256), 256, 128),
+    (256, (256, 257, 384, 385, 512, 640), 512, 128),
+    (0, (300,) * 20 + (100,) * 44, 256, 2048), (0, (17, 200, 256, 31) * 8, 512, 640),
+    (128, (1025, 1056, 1057, 1088, 1152, 1153, 1024, 897), 256, 1024),
+    (128, (1025, 1056, 1057, 1281, 1152, 1409, 1024, 0), 256, 1024)])
+def test_gemm_tiles_at_their_edges(gpu_sa, narrow, counts, K, N):
     """Wide and narrow tiles of every filling (row blocks of one or both wave
-    halves, DMA groups partly past the last pair, short last tiles narrow or
-    wide, every tile narrow), as chosen and with 256- and 128-pair tiles: the
-    same MFMA sequence per output element, so the same bits; and the oracle."""
+    halves, DMA groups partly past the last pair, every tile narrow, every tile
+    wide, and wide tiles with the short last ones of an expert narrow: 1 to 128
+    pairs, 129 wide, none after a multiple of 256, an empty expert), as chosen
+    and with 256- and 128-pair tiles: the same MFMA sequence per output element,
+    so the same bits; and the oracle."""
     E, M = len(counts), sum(counts)
+    p = moe_plan(M, K, N, E, 1)
+    assert p["gemm"] and p["tile_rows"] == 256 and p["narrow_rows"] == narrow
     hidden, w1, w2, _ = make_inputs(M, K, N, E, seed=11)
     ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
     ids = ids[torch.randperm(M, generator=torch.Generator().manual_seed(12))].to(DEV)
@@ -217,6 +223,9 @@ def test_gemm_silu_of_every_bf16_gate(gpu_sa, flags):
     w1 = torch.cat([x, torch.ones_like(x)])[None].to(DEV)
     eye = torch.eye(n, dtype=torch.bfloat16, device=DEV)
     score = torch.zeros(n, 1, dtype=torch.bfloat16, device=DEV)
+    p = moe_plan(n, n, n, 1, 1, flags)
+    assert (p["gemm"], p["tile_rows"], p["narrow_rows"]) == \
+        (1, *{0: (256, 256), 1: (128, 0), 4: (256, 0)}[flags])
     got = op(eye, w1, eye[None].contiguous(), score, 1, flags=flags)
     streamed = op(eye, w1, eye[None].contiguous(), score, 1, flags=2 | 8)
     bad = torch.nonzero(got.t().cpu().view(torch.int16) != streamed.t().cpu().view(torch.int16))
