@@ -40,10 +40,14 @@ def run(q, kv, sink, idx, scale, flags=0):
 
 
 # (b, m, kv_len, topk, flags, minus1): a per-query plan, forced shared-row
-# tiles with -1 padding, and a split-topk (decode) plan
+# tiles with -1 padding, a split-topk (decode) plan, and long caches with four,
+# two and one waves per query
 PLANS = {"per query": (1, 300, 5000, 128, PER_QUERY, 0.0),
          "tiles": (2, 24, 700, 96, FORCE_TILES, 0.2),
-         "split": (4, 1, 9000, 1500, 0, 0.1)}
+         "split": (4, 1, 9000, 1500, 0, 0.1),
+         "4 waves": (2, 150, 16400, 500, 0, 0.1),
+         "2 waves": (1, 520, 16400, 1100, 0, 0.1),
+         "1 wave": (1, 1540, 16400, 400, 0, 0.1)}
 
 
 @pytest.mark.parametrize("h", [1, 2, 4, 8, 32, 48])

@@ -1,7 +1,9 @@
 """GPU parity of the one-wave-per-query kernel (sa_fwd_wave_kernel): short
 unsplit queries (topk <= 384) of per-query plans and of the per-query tiles
 of shared-row plans, checked against the float64 oracle on every query, with
-the launched-kernel mask of sa_forward_events naming the kernel that ran.
+the launched-kernel mask of sa_forward_events naming the kernel that ran; and
+of the kernel with W waves per query (sa_fwd_waves_kernel): unsplit queries of
+385 to 2 048 slots over caches too long for shared tiles.
 
 Tolerance as in test_gpu_parity: max |err| <= 2e-2, mean |err| <= 2e-3,
 relative RMS <= 5e-3 against float64; lse max |err| <= 2e-3; exact zeros for
@@ -67,7 +69,7 @@ def per_query_queries(ws, b, m):
 # plan does not split them (asserted first).
 @pytest.mark.parametrize("b,m,kv_len,topk,minus1", [
     (2, 160, 1024, 128, 0.0),    # contest-like prefill: every tile per query
-    (1, 261, 4096, 100, 0.2),    # ragged last tile (5 queries: a one-query work-group)
+    (1, 261, 4096, 100, 0.2),    # ragged last tile (5 queries)
     (3, 89, 2048, 384, 0.1),     # the largest list; tiles of 8 + 1
     (1, 24, 600, 17, 0.0),       # one 16-row and one 1-row step (tiles shared here)
     # a batch's kv above 4 MiB: each query's rows sorted ascending (2, 4 and
@@ -100,10 +102,9 @@ def test_wave_tiles_full(gpu_sa, b, m, kv_len, topk, minus1):
 
 @pytest.mark.parametrize("b,m", [(3, 99), (5, 61)])
 def test_wave_plain_plan_across_batches(gpu_sa, b, m):
-    """The plain per-query plan: work-group i runs queries 2i and 2i + 1 of
-    b x m, which straddle batches when m is odd; the last work-group has one
-    query. Different kv per batch, so a query gathered from the wrong batch
-    fails the oracle check."""
+    """The plain per-query plan: work-group i runs query i of b x m. Different
+    kv per batch, so a query gathered from the wrong batch fails the oracle
+    check."""
     q, kv, sink, idx, sc = case(b, m, 777, 200, seed=b + m, minus1=0.05)
     p = expect_plan(q, kv, idx, PER_QUERY, tiles=False)
     if p["nsplit"] != 1:
@@ -339,3 +340,37 @@ def test_long_cache_rows_whose_scores_overflow(gpu_sa, m, topk):
     o_ref, lse_ref = sparse_attn_lse_fp64(q[:, sel], kv, sink, ref[:, sel], sc)
     check(o.cpu()[:, sel], o_ref, f"overflowing scores, topk {topk}")
     assert np.abs(lse.double().cpu().numpy()[:, sel] - lse_ref).max() <= 2e-3
+
+
+@pytest.mark.parametrize("m,topk", LONG_CACHE)
+def test_long_cache_waves_strided(gpu_sa, m, topk):
+    """Strided q, kv (rows and batches), idx, o and lse: the contiguous call's
+    bits, and nothing written into the gaps."""
+    q, kv, sink, idx, sc = (t.to(DEV) if torch.is_tensor(t) else t
+                            for t in case(2, m // 2, 16400, topk, seed=topk + 2, minus1=0.1))
+    b, m = q.shape[:2]
+    if expect_plan(q, kv, idx, 0, tiles=False)["nsplit"] != 1:
+        pytest.skip("split on this device")
+    o_ref, lse_ref, mask, _, _ = run(q, kv, sink, idx, sc, with_lse=True)
+    assert mask == QUERY
+    nan = float("nan")
+    qs = torch.full((b, m, 32, 520), nan, dtype=torch.bfloat16, device=DEV)[:, :, ::2, :512]
+    kvs = torch.full((b, 16500, 584), nan, dtype=torch.bfloat16, device=DEV)[:, 50:16450, :512]
+    idxs = torch.full((m, b, 2 * topk), -1, dtype=torch.int32, device=DEV)
+    idxs = idxs.transpose(0, 1)[..., :topk]
+    qs.copy_(q), kvs.copy_(kv), idxs.copy_(idx)
+    o_base = torch.full((b, m, 32, 576), nan, dtype=torch.bfloat16, device=DEV)
+    lse_base = torch.full((b, m, 32), nan, device=DEV)
+    o, lse = o_base[:, :, ::2, :512], lse_base[:, :, ::2]
+    lib = sa_capi.load()
+    a = sa_capi.make_args(qs, kvs, sink, idxs, o, sc, 0, lse=lse)
+    n = sa_capi.workspace_bytes(lib, a)
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=DEV)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n
+    mask = sa_capi.forward_events(lib, a, torch.cuda.current_stream().cuda_stream,
+                                  [None] * (2 * sa_capi.SA_KERNEL_COUNT))
+    torch.cuda.synchronize()
+    assert mask == QUERY
+    assert torch.equal(o, o_ref) and torch.equal(lse, lse_ref)
+    assert o_base[:, :, 1::2].isnan().all() and o_base[..., 512:].isnan().all()
+    assert lse_base[:, :, 1::2].isnan().all()
