@@ -50,9 +50,9 @@ enum {
   FM_FLAG_ORDERED_SUM = 8u   /* (ABI version 4) the final sum over a token's experts
                                 always runs as its own launch (the ascending-expert
                                 running bf16 sum), never as the down GEMM's bf16
-                                atomic adds into the output (topk <= 2 with up to
-                                24 pairs per expert); the result is the same bits.
-                                Combines with one tile flag. */
+                                atomic adds into the output (see FM_KERNEL_REDUCE);
+                                the result is the same bits. Combines with one tile
+                                flag. */
 };
 
 typedef struct fm_args {
@@ -91,9 +91,10 @@ enum {
   FM_KERNEL_GATEUP = 2,  /* x = h . w1^T, u = up * silu(gate)        */
   FM_KERNEL_DOWN = 3,    /* y = u . w2^T, times the routing weight   */
   FM_KERNEL_REDUCE = 4,  /* ascending-expert bf16 sum per token; since
-                            version 3 not launched for topk <= 2 with up
-                            to 24 pairs per expert (decode): the down
-                            GEMM adds into out itself                */
+                            version 3 not launched for topk <= 2 and N
+                            a multiple of 256 with up to 24 pairs per
+                            expert (decode) or FM_FLAG_SMALL_TILES: the
+                            down GEMM adds into out itself           */
   FM_KERNEL_COUNT = 5
 };
 

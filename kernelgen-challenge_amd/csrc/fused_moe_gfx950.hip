@@ -34,8 +34,8 @@
 //   and the 4 waves of a work-group split K and add their partial sums
 //   through LDS. 16x16x32 bf16 MFMA.
 // fm_reduce_kernel  out[t] = bf16 running sum of the token's topk weighted
-//   expert outputs, ascending expert order. Not launched when topk <= 2 and
-//   experts have few pairs (decode): the routing launch clears out, and the
+//   expert outputs, ascending expert order. Not launched when topk <= 2, N % 256
+//   == 0 and experts have few pairs (decode): the routing launch clears out, and the
 //   down GEMM adds each weighted row into it with packed bf16 atomics (the
 //   two-term bf16 sum does not depend on the order).
 #include <hip/hip_ext.h>
@@ -699,7 +699,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* s_buf, i
   float wt[kRB];
   if constexpr (!kGated && NRB > 0) {
 #pragma unroll
-    for (int rb = 0; rb < NRB; ++rb) 
+    for (int rb = 0; rb < NRB; ++rb)
       pair[rb] = p.sorted[start + min(32 * (kPh * rb + ph) + l32, rows - 1)];
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb) wt[rb] = p.wts[pair[rb]];
@@ -722,8 +722,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* s_buf, i
     if (f < 2)
       fr.b[f] = *reinterpret_cast<const bf16x8*>(sb + (64 * wq + 32 * f + l32) * kRowBytes + pos);
     else if (f - 2 < NRB)
-      fr.a[f - 2] =
-          *reinterpret_cast<const bf16x8*>(
+      fr.a[f - 2] = *reinterpret_cast<const bf16x8*>(
           sa + (32 * (kPh * (f - 2) + ph) + l32) * kRowBytes + pos);
   };
   // The MFMAs of step (fr), with the reads of the next step (sa, sb, kk) into
@@ -815,8 +814,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* s_buf, i
   }
 
   // epilogue: the lane holds, for pair row 32 * (kPh * rb + ph) + l32, weight
-  // rows
-  // 8 * a + 4 * hi + i of each column block in register 4 * a + i. The outputs
+  // rows 8 * a + 4 * hi + i of each column block in register 4 * a + i. The outputs
   // go through this wave's own LDS lines, so that global stores write 64
   // (gated) or 128 contiguous bytes of a row by 16 bytes per lane: 2 us instead
   // of 5 for 2-byte stores straight from the accumulators.
@@ -1307,9 +1305,9 @@ int forward(const fm_args* a, hipStream_t stream, void* const* events, uint32_t*
   rp.E = int(a->E);
   rp.topk = int(a->topk);
   rp.renormalize = a->renormalize ? 1 : 0;
-  // With at most two experts per token, the down GEMM of streamed tiles, or of
-  // up to 24 pairs per expert, adds into the output itself and the routing
-  // launch clears it: no final-sum launch.
+  // With at most two experts per token and N a multiple of kStK, the down GEMM
+  // of streamed tiles, or of up to 24 pairs per expert, adds into the output
+  // itself and the routing launch clears it: no final-sum launch.
   const bool streamed = !pl.gemm && a->N % kStK == 0;  // (K % 256 == 0 always holds)
   const bool fsum = a->topk <= 2 && (a->flags & FM_FLAG_ORDERED_SUM) == 0 &&
                     (streamed || (pl.gemm && a->N % kStK == 0 && pl.P <= 24 * a->E));

@@ -119,7 +119,11 @@ constexpr int kTQ = sa::kTileQueries;       // queries per shared tile
 // many), the per-query launch's time adds to the slowest tile's instead of
 // filling in behind other tiles, and its work-groups have a CU each: a query
 // is priced at 4 900 plus 35 per slot. (At the lower price high locality's
-// longest tiles went per query and the call took 134 us instead of 116.)
+// longest tiles went per query and the call took 134 us instead of 116.) These
+// two are figures of the 4-wave kernel (topk 512) and hold for every topk there,
+// too dear where one wave runs a query (topk <= kWaveMaxTopk): every tile
+// shared / every query per query, 16 x 128 queries, kv_len 1 024, topk 128 58 / 40
+// us, topk 300 72 / 75; 4 x 512, windows of 16 384, topk 256 73 / 70.
 constexpr int64_t kSharedTileNs = 10000;
 constexpr int64_t kSharedPairNs10 = 66;   // x 10
 constexpr int64_t kQueryUnitNs = 2100;
@@ -127,13 +131,12 @@ constexpr int64_t kQuerySlotNs = 27;
 // Queries of topk <= kWaveMaxTopk run one wave each: 1 350 plus 12 per slot (64
 // x 1024 queries, kv_len 1 024 and 1 280, topk 128, 200 and 384), or 22 where
 // a batch's kv exceeds an XCD's L2 (topk 128 at 16 384, 300 at 20 480). Whole
-// calls, tiles shared -> per query: 64 x 1024, kv_len 1 280, topk 384 2 377 ->
-// 1 511 us; 64 x 512, 512, 128 578 -> 381; 64 x 1024, 600, 256 1 411 -> 1 144;
-// causal 4 096, topk 256 122 -> 100. The pair-skipping form of the shared tiles
-// (kTQ * topk < kv_len) costs about 4.5 per pair where queries share windows
-// of rows; priced at 6.6 against the wave's figures, such tiles went per query
-// too early: 4 x 4096, kv_len 8 192, topk 256 470 -> 514 us; 2 x 2000, 16 384,
-// 320 186 -> 222.
+// calls, every tile shared / as priced: 64 x 1024, kv_len 1 280, topk 384 2 380 /
+// 1 498 us; 64 x 512, 512, 128 573 / 362; 64 x 1024, 600, 256 1 389 / 1 120;
+// causal 4 096, topk 256 194 / 107. The pair-skipping form of the shared tiles
+// (kTQ * topk < kv_len) costs about 4.5 per pair where queries share windows of
+// rows: 4 x 4096, kv_len 8 192, topk 256 442 / 453; 2 x 2000, 16 384, 320 147 /
+// 173. (At 6.6 more of those tiles went per query: 514 and 222.)
 constexpr int64_t kWaveUnitNs = 1350;
 constexpr int64_t kWaveSlotNs = 12;
 constexpr int64_t kWaveFarSlotNs = 22;
@@ -299,18 +302,6 @@ __device__ __forceinline__ void mfma_agpr(f32x16& c, bf16x8 a, bf16x8 b) {
       "v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
       : "+a"(c)
       : "v"(a), "v"(b));
-}
-
-// v_mfma_f32_16x16x32_bf16 accumulating in VGPRs with its B operand in
-// AGPRs (an operand that lives in AGPRs for good, such as a resident Q^T,
-// then takes no VGPRs). The same hazards; the VALU reads of the result wait
-// for mfma_agpr_drain().
-__device__ __forceinline__ void mfma32_bagpr(f32x4& c, bf16x8 a, const bf16x8& b) {
-  asm volatile(
-      "s_nop 1\n\t"
-      "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-      : "+v"(c)
-      : "v"(a), "a"(b));
 }
 
 __device__ __forceinline__ f32x4 mfma_16x16x16(bf16x4 a, bf16x4 b, f32x4 c) {
@@ -3341,12 +3332,14 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
   p.split_len = plan.split_len;
   p.nblocks = plan.units * plan.nsplit;
   // the wave kernel sorts its queries' rows when a batch's kv span exceeds an
-  // XCD's L2 (from the shape alone, so every path of a call sorts alike)
+  // XCD's L2 (from kv_len and the row stride, so every path of a call sorts
+  // alike)
   p.sort_wave = int64_t(a->kv_len) * a->skv[1] * 2 > kWaveSortBytes ? 1 : 0;
 
   // Short unsplit queries run one wave each (sa_fwd_wave_kernel): its list
-  // holds 32-bit row offsets in a batch of kv. (Its epilogue's bf16 pair
-  // stores need o 4-byte aligned: validate() asks for 16.)
+  // holds 32-bit row offsets in a batch of kv. (It stores o by 16 bytes per
+  // lane: validate() asks for that alignment and strides that are multiples of
+  // 8 elements.)
   const bool wave_ok =
       what == Launch::kCall && plan.nsplit == 1 && a->topk <= kWaveMaxTopk && a->kv_len > 0 &&
       (a->kv_len - 1) * a->skv[1] * 2 + 2 * kDim <= int64_t(UINT32_MAX);
@@ -3402,7 +3395,8 @@ int forward16(const sa_args* a, hipStream_t stream, void* const* events, uint32_
     ip.force = (a->flags & SA_FLAG_FORCE_TILES) ? 1 : 0;
     ip.vec4 = ((reinterpret_cast<uintptr_t>(a->idx) & 15u) == 0 && a->topk % 4 == 0 &&
                a->sidx[0] % 4 == 0 && a->sidx[1] % 4 == 0) ? 1 : 0;
-    // from the shape alone, so that an index plan makes the plain call's modes
+    // from the shape and kv's row stride, which an index plan is made for, so
+    // that it makes the plain call's modes
     const bool placed_regime = 2 * plan.ntiles >= cus && plan.ntiles <= cus;
     const bool waves = a->topk <= kWaveMaxTopk;  // one wave per query
     ip.pair_ns10 = int(waves && !placed_regime && kTQ * a->topk < a->kv_len ? kSharedSkipPairNs10

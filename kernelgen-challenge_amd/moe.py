@@ -9,7 +9,7 @@ in the operator) and the output is a new ``[M, K]`` tensor of
 ``track-03/reference/reference.py:10-35`` with its bf16 rounding points,
 including ``renormalize`` (which the reference's Triton submission ignores,
 ``:276-277``). Ties in the top-k go to the lower expert index (the
-reference leaves them to ``torch.topk``). Five HIP kernel launches
+reference leaves them to ``torch.topk``). Three to five HIP kernel launches
 (``csrc/fused_moe_gfx950.hip`` behind ``include/fused_moe.h``) on the
 current stream, with no synchronisation; the workspace comes from torch's
 caching allocator. There is no CPU path: CPU tensors raise ``ValueError``.

@@ -120,7 +120,7 @@ def test_wave_plain_plan_across_batches(gpu_sa, b, m):
 def test_wave_masked_duplicates_and_sink(gpu_sa):
     """Queries with no valid slot give exact zeros (lse = the sink's), all-
     duplicate queries weigh one row by its count, and -1 slots anywhere are
-    skipped, all within one two-query work-group's stream."""
+    skipped."""
     q, kv, sink, idx, sc = case(1, 16, 512, 48, seed=3)
     idx[0, 0] = -1                                      # nothing valid
     idx[0, 1, :] = 7                                    # one row, 48 times
